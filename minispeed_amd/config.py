@@ -19,9 +19,9 @@ One section is specific to this package and ignored by minispeed:
                      "state_spacing_gib": "auto", "stage3_gather_reuse": false}
 
 With ``materialize_flat_grad`` the ragged-grad kernel also writes the fp32
-flat gradient buffer and the AdamW kernel reads it back (36 B/param for half
-grads); by default the AdamW kernel re-reads the ragged half gradients and
-the flat buffer is never written (30 B/param).  Both give identical results.
+flat gradient buffer (34 B/param for half grads); by default the flat buffer
+is never written (30 B/param).  The AdamW kernel reads the ragged gradients
+either way.  Both give identical results.
 
 ``contiguous_gradients`` (opt-in) accumulates every micro-batch gradient in
 fp32 straight into a flat buffer as backward produces it, instead of in the

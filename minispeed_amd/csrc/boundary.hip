@@ -150,7 +150,9 @@ constexpr int64_t kXcdChunk = MS_XCD_CHUNK;
 // params 0.636 -> 0.618 ms, 350M 1.714 -> 1.694, 1.3B 6.228 -> 6.198 (K3
 // 5.792 -> 5.763, K1 +6 us); 96 / 160 / 224 / 320 MiB / every run: 124M
 // 0.634 / 0.627 / 0.619 / 0.620 / 0.619 ms, 1.3B 6.22 / 6.21 / 6.198 /
-// 6.200 / 6.237 (ordinary loads throughout slow K1 by 40 us there).
+// 6.200 / 6.237 (ordinary loads throughout slow K1 by 40 us there).  Writing
+// the flat gradient too, K1 does the same for the same tiles (K3 reads the
+// gradients, not their fp32 copy): 350M fp16 params 1.949 -> 1.922 ms a step.
 #ifndef MS_CACHE_KEEP_MIB
 #define MS_CACHE_KEEP_MIB 224
 #endif
@@ -689,7 +691,7 @@ constexpr int scan_min_waves() { return kFlat ? MS_SCAN_MIN_WAVES_FLAT : MS_SCAN
 // wave 0 adds the squares in the walk's order: lane l its head element,
 // its tail element, then units l, l + 64, ..., so the slot gets the bits
 // one wave alone gives it.
-template <class Scan, class G, bool kStats, int kScale, int kWaves>
+template <class Scan, class G, bool kStats, int kScale, int kWaves, bool kKeep>
 __device__ void split_tile_shifted(Scan& sc, const ms_segment_t& sg, int64_t r0, int64_t begin,
                                    int m, bool owned, float* __restrict__ flat, int64_t t,
                                    double* __restrict__ tsum, uint32_t* __restrict__ tflag,
@@ -708,7 +710,7 @@ __device__ void split_tile_shifted(Scan& sc, const ms_segment_t& sg, int64_t r0,
 #pragma unroll
   for (int k = 0; k < kPerLane; ++k) {
     const int u = (wave * kPerLane + k) * 64 + lane;
-    if (u < kUnits) load_unit(usrc + static_cast<int64_t>(u) * 16, w[k]);
+    if (u < kUnits) load_unit<kKeep>(usrc + static_cast<int64_t>(u) * 16, w[k]);
   }
   // head (wave 0, lanes < nh) and tail (wave 1, lanes < m) elements
   bool ebad = false;
@@ -814,8 +816,8 @@ __device__ void scan_tile(Scan& sc, const ms_segment_t* segs, int nseg, int& s, 
 // Reading only (kFlat false): each wave scans runs of `run` consecutive
 // tiles; a run starting at tile keep_from or later is loaded with ordinary
 // loads (kCacheKeepBytes).  Writing the flat gradient (kFlat): one block of kScanWavesFlat
-// waves per tile.  A whole tile inside one segment with 16-byte aligned
-// storage, starting on a unit boundary of it and owned or not as a whole,
+// waves per tile, the tiles from keep_from on loaded with ordinary loads.  A
+// whole tile inside one segment with 16-byte aligned storage, starting on a unit boundary of it and owned or not as a whole,
 // is split across the waves: wave w loads, widens and writes units
 // w*k*64 + lane .. (k units per lane), each store covering whole lines; the
 // widened values wait in LDS, and after a barrier wave 0 adds each lane's
@@ -884,7 +886,9 @@ __global__ __launch_bounds__(64 * scan_waves<kFlat>(), scan_min_waves<kFlat>()) 
     // current tile's loads are in flight (a block takes its tiles one after
     // another, so the search would otherwise add to every tile's time)
     int snext = tfirst < ntiles ? find_seg(segs, nseg, begin + tfirst * kScanTile) : 0;
-    for (int64_t t = tfirst; t < ntiles; t += gridDim.x) {
+    // one tile; the load hint is a compile-time choice, as when reading
+    auto tile = [&](int64_t t, auto keep) {
+      constexpr bool kKeep = decltype(keep)::value;
       Scan sc;
       sc.mul = mul;
       sc.div = div;
@@ -909,23 +913,23 @@ __global__ __launch_bounds__(64 * scan_waves<kFlat>(), scan_min_waves<kFlat>()) 
           scan_tile<Scan, G, kStats>(sc, segs, nseg, s, t, r0, r1, own_begin, own_end, tsum,
                                      tflag, lane);
         if (tn < ntiles) snext = find_seg(segs, nseg, begin + tn * kScanTile);
-        continue;
+        return;
       }
       // the tile's first element sits m elements into a unit of the storage
       const int m = static_cast<int>((r0 - sg.begin) & (kUnit - 1));
       if (m != 0) {
-        split_tile_shifted<Scan, G, kStats, kScale, kWaves>(
+        split_tile_shifted<Scan, G, kStats, kScale, kWaves, kKeep>(
             sc, sg, r0, begin, m, owned, flat, t, tsum, tflag, (MS_LDS float*)&slabs[0][0],
             (MS_LDS uint32_t*)wflag, wave, lane, mul, div);
         if (tn < ntiles) snext = find_seg(segs, nseg, begin + tn * kScanTile);
         __syncthreads();   // the staged tile and flags are rewritten by the next tile
-        continue;
+        return;
       }
       const char* src = static_cast<const char*>(sg.grad) + (r0 - sg.begin) * G::kBytes;
       uint32_t w[kPerLane][4];
 #pragma unroll
       for (int k = 0; k < kPerLane; ++k)
-        load_unit(src + ((wave * kPerLane + k) * 64 + lane) * 16, w[k]);
+        load_unit<kKeep>(src + ((wave * kPerLane + k) * 64 + lane) * 16, w[k]);
       if (tn < ntiles) snext = find_seg(segs, nseg, begin + tn * kScanTile);
       float g[kPerLane][kUnit];
 #pragma unroll
@@ -988,6 +992,12 @@ __global__ __launch_bounds__(64 * scan_waves<kFlat>(), scan_min_waves<kFlat>()) 
         }
         __syncthreads();   // the slabs and flags are rewritten by the next tile
       }
+    };
+    for (int64_t t = tfirst; t < ntiles; t += gridDim.x) {
+      if (kStats && t >= keep_from)
+        tile(t, BoolC<true>{});
+      else
+        tile(t, BoolC<false>{});
     }
   }
 }
@@ -1563,18 +1573,18 @@ template <class G, int kScale>
 void launch_stats_s(const ms_segment_t* segs, int nseg, int64_t begin, int64_t end, int64_t ob,
                     int64_t oe, float mul, float div, float* flat, double* tsum, uint32_t* tflag,
                     int64_t ntiles, hipStream_t st) {
+  // the tiles holding the last kCacheKeepBytes of gradient
+  const int64_t keep_tiles = kCacheKeepBytes / (int64_t(kScanTile) * G::kBytes);
+  const int64_t keep_from = ntiles > keep_tiles ? ntiles - keep_tiles : 0;
   if (tsum) {
     if (flat) {
       hipLaunchKernelGGL((k_grad_stats<G, true, true, kScale>), dim3(scan_grid(ntiles, 1)),
                          dim3(64 * kScanWavesFlat), 0, st, segs, nseg, begin, end, ob, oe, mul,
-                         div, flat, tsum, tflag, ntiles, 1, ntiles);
+                         div, flat, tsum, tflag, ntiles, 1, keep_from);
     } else {
       // runs of 2 and 4 tiles time alike over 60K-640K tiles, runs of 1 up
       // to 30% slower
       constexpr int kRun = MS_SCAN_RUN_READ;
-      // the tiles holding the last kCacheKeepBytes of gradient
-      const int64_t keep_tiles = kCacheKeepBytes / (int64_t(kScanTile) * G::kBytes);
-      const int64_t keep_from = ntiles > keep_tiles ? ntiles - keep_tiles : 0;
       // the counted elements' flags from their sums wherever the scaling
       // cannot overflow a finite gradient (GradScan's kSumFlags)
       const bool sum_flags = kScale == kScaleNone ||
