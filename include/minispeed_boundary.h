@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MS_ABI_VERSION 8
+#define MS_ABI_VERSION 9
 
 /* groups one ms_boundary_scalars_noalloc call can scan, and the tiles
  * (MS_SCAN_TILE flat indices each) of the largest one: its static scratch
@@ -219,6 +219,42 @@ int ms_norm_clip(const double* block_sumsq, const uint32_t* block_flag,
                  int64_t good_steps, int64_t skipped_steps, int64_t window,
                  double min_scale, double max_scale, ms_step_scalars_t* out,
                  ms_step_scalars_t* out_host, void* stream);
+
+/* K1 without the fold: ms_grad_stats writing the tile slots only (required
+ * here), for ms_norm_clip_tiles. */
+int ms_grad_tile_stats(const ms_segment_t* segs, int32_t nseg, int32_t grad_dtype,
+                       int64_t begin, int64_t end, int64_t own_begin, int64_t own_end,
+                       int32_t unscale, float grad_scale, float* flat_grad,
+                       double* tile_sumsq, uint32_t* tile_flag, int64_t ntiles,
+                       void* stream);
+
+/* The tile statistics of one group: ntiles slots [dev] that K1
+ * (ms_grad_tile_stats) or K5 (ms_accumulate_grads) wrote.  The pointers may
+ * be NULL when ntiles is 0 (a group that adds nothing). */
+typedef struct ms_tile_stats {
+  const double* sumsq;
+  const uint32_t* flag;
+  int64_t ntiles;
+} ms_tile_stats_t;
+
+/* groups whose tiles K2 can read itself (their descriptors travel in its
+ * kernel arguments); the later groups of a call are folded first */
+#define MS_NORM_DIRECT_GROUPS 8
+
+/*
+ * ms_reduce_tile_stats of every group, then ms_norm_clip, bit for bit; a
+ * group of at most ms_stats_blocks() tiles is read by K2 straight from its
+ * tile slots, without the fold's launch.
+ * groups [host]: ngroups entries.  block_sumsq / block_flag [dev]: workspace
+ *   of ngroups x nblk slots (nblk >= ms_stats_blocks()) for the folds.  The
+ *   other arguments are ms_norm_clip's.
+ */
+int ms_norm_clip_tiles(const ms_tile_stats_t* groups, int32_t ngroups, double* block_sumsq,
+                       uint32_t* block_flag, int32_t nblk, int32_t has_clip,
+                       double max_norm, int32_t scaler_enabled, double scale,
+                       int64_t good_steps, int64_t skipped_steps, int64_t window,
+                       double min_scale, double max_scale, ms_step_scalars_t* out,
+                       ms_step_scalars_t* out_host, void* stream);
 
 /*
  * K3 — fused AdamW over the owned range [begin, end) plus the cast of the

@@ -19,7 +19,7 @@ from typing import Optional
 import torch  # noqa: F401  (must precede the dlopen below, see module doc)
 
 LIB_NAME = "libminispeed_boundary.so"
-ABI_VERSION = 8
+ABI_VERSION = 9
 
 DTYPE_F32 = 0
 DTYPE_F16 = 1
@@ -101,6 +101,16 @@ class GroupScan(ctypes.Structure):
     ]
 
 
+class TileStats(ctypes.Structure):
+    """``ms_tile_stats_t``: one group of ms_norm_clip_tiles."""
+
+    _fields_ = [
+        ("sumsq", ctypes.c_void_p),
+        ("flag", ctypes.c_void_p),
+        ("ntiles", ctypes.c_int64),
+    ]
+
+
 class AccumRow(ctypes.Structure):
     """``ms_accum_row_t``: one gradient of ms_accumulate_grads."""
 
@@ -140,6 +150,15 @@ SIGNATURES = {
     "ms_norm_clip": (
         ctypes.c_int,
         [_P, _P, _I32, _I32, _I32, _D, _I32, _D, _I64, _I64, _I64, _D, _D, _P, _P, _P],
+    ),
+    "ms_grad_tile_stats": (
+        ctypes.c_int,
+        [_P, _I32, _I32, _I64, _I64, _I64, _I64, _I32, _F, _P, _P, _P, _I64, _P],
+    ),
+    "ms_norm_clip_tiles": (
+        ctypes.c_int,
+        [ctypes.POINTER(TileStats), _I32, _P, _P, _I32, _I32, _D, _I32, _D, _I64, _I64, _I64, _D, _D,
+         _P, _P, _P],
     ),
     "ms_fused_adamw": (
         ctypes.c_int,

@@ -124,12 +124,13 @@ class Workspace:
         self.partials = torch.empty(n, dtype=torch.float64, device=device)
         self.flags = torch.empty(n, dtype=torch.int32, device=device)
         self.scalars = torch.empty(_native.SCALARS_BYTES, dtype=torch.uint8, device=device)
-        # K1's tile slots, shared by the groups of a boundary (each group's
-        # K1 and fold run before the next group's K1, on one stream); grown
+        # K1's tile slots, the groups of a boundary one after another; grown
         # on demand, with every stream that used them recorded
         self.tile_sums: Optional[torch.Tensor] = None
         self.tile_flags: Optional[torch.Tensor] = None
         self._tile_streams: set = set()
+        # every group's tile statistics, filled in for each call of K2
+        self.tile_stats = (_native.TileStats * max(1, ngroups))()
         # K2 also writes its result to pinned host memory, which the host
         # polls (HostReadback): no copy, and K3, queued behind K2, keeps
         # running while the host does its bookkeeping
@@ -294,9 +295,9 @@ def run_boundary(
 ) -> _native.StepScalars:
     """Launch the whole boundary and return K2's scalars (one host sync).
 
-    K1 and K2 are launched as soon as the gradient addresses are known (K2
-    writes its scalars to device memory for K3 and to pinned host memory
-    for the host) and an event marks K2's end; ``model_targets()``
+    K1 per group and K2 with the folds it needs are launched as soon as the
+    gradient addresses are known (K2 writes its scalars to device memory for
+    K3 and to pinned host memory for the host); ``model_targets()``
     (the addresses K3 casts the updated masters into, per group; ``None`` for
     no write) is called after that, so whatever it does on the host overlaps
     K1 on the device.  The function returns once K2's scalars are on the
@@ -316,6 +317,15 @@ def run_boundary(
     timer = timer or _NO_TIMER
 
     dtypes = []
+    # a group whose accumulation pass already scanned the sums has its tile
+    # statistics (no second read of the sums); the others' tile slots lie one
+    # region after another, K2 reads them all
+    scanned = [gl.tile_stats is not None and not materialize_flat_grad
+               and gl.group.own_range == (0, gl.group.numel_padded) for gl in launches]
+    ntiles = [0 if done else _native.scan_tiles(gl.group.numel_padded)
+              for gl, done in zip(launches, scanned)]
+    tsum, tflag = ws.tile_ptrs(sum(ntiles))
+    stats = ws.tile_stats
     for gi, gl in enumerate(launches):
         g = gl.group
         dtype = _native.ms_dtype(g.params[0].dtype)
@@ -325,34 +335,30 @@ def run_boundary(
             flat_out = g.flat_grad_for_overwrite()      # K1 writes every element
         lo, hi = g.own_range
         gbytes = 4 if gdtype == _native.DTYPE_F32 else 2
-        psum, pflag = ws.partial_ptrs(gi)
-        if gl.tile_stats is not None and flat_out is None and (lo, hi) == (0, g.numel_padded):
-            # the accumulation pass already scanned the sums: fold its tile
-            # statistics into the partial slots (no second read of the sums)
-            ts, tf, ntiles = gl.tile_stats
-            tok = timer.start("k1")
-            rc = lib.ms_reduce_tile_stats(ts or None, tf or None, ntiles, psum, pflag, ws.nblk, stream)
+        if scanned[gi]:
+            tok = timer.start("k1")          # nothing to launch
+            stats[gi].sumsq, stats[gi].flag, stats[gi].ntiles = gl.tile_stats
             timer.stop(tok)
-            _native.check(rc, "ms_reduce_tile_stats")
         else:
             t1 = g.table("k1").upload(g.boundary_table(0, g.numel_padded, gl.grads, None, gbytes), cur)
-            ntiles = _native.scan_tiles(g.numel_padded)
-            tsum, tflag = ws.tile_ptrs(ntiles)
             tok = timer.start("k1")
-            rc = lib.ms_grad_stats(
+            rc = lib.ms_grad_tile_stats(
                 t1[0], t1[1], gdtype, 0, g.numel_padded, lo, hi,
                 _native.SCALE_DIVIDE if unscale else _native.SCALE_NONE, scale32,
                 flat_out.data_ptr() if flat_out is not None else None,
-                tsum, tflag, ntiles, psum, pflag, ws.nblk, stream,
+                tsum, tflag, ntiles[gi], stream,
             )
             timer.stop(tok)
-            _native.check(rc, "ms_grad_stats")
+            _native.check(rc, "ms_grad_tile_stats")
+            stats[gi].sumsq, stats[gi].flag, stats[gi].ntiles = tsum, tflag, ntiles[gi]
+            tsum += 8 * ntiles[gi]
+            tflag += 4 * ntiles[gi]
         dtypes.append((gdtype, dtype, gbytes))
 
     ws.readback.arm()
     tok = timer.start("k2")
-    rc = lib.ms_norm_clip(
-        ws.partials.data_ptr(), ws.flags.data_ptr(), ws.nblk, len(launches),
+    rc = lib.ms_norm_clip_tiles(
+        stats, len(launches), ws.partials.data_ptr(), ws.flags.data_ptr(), ws.nblk,
         1 if max_norm is not None else 0, float(max_norm or 0.0),
         1 if scaler.enabled else 0, float(scaler.scale), int(scaler.good_steps),
         int(scaler.skipped_steps), int(scaler.scale_window),
@@ -360,7 +366,7 @@ def run_boundary(
         ws.scalars.data_ptr(), ws.readback.ptr, stream,
     )
     timer.stop(tok)
-    _native.check(rc, "ms_norm_clip")
+    _native.check(rc, "ms_norm_clip_tiles")
 
     models = model_targets()
     for gl, (gdtype, dtype, gbytes), mptrs in zip(launches, dtypes, models):

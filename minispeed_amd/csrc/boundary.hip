@@ -117,6 +117,8 @@ constexpr int kScanTile = MS_SCAN_TILE;
 #ifndef MS_SCAN_DEPTH_FLAT
 #define MS_SCAN_DEPTH_FLAT 1
 #endif
+// 256 CUs x 3 blocks of 8 waves hold 6144 waves of the reading K1 at a time
+constexpr int64_t kShortScanTiles = 6144;
 constexpr int kScanWavesRead = MS_SCAN_WAVES_READ;
 constexpr int kScanWavesFlat = MS_SCAN_WAVES_FLAT;
 // waves per SIMD K1 is compiled for: left alone, the compiler widens every
@@ -158,6 +160,7 @@ constexpr int64_t kXcdChunk = MS_XCD_CHUNK;
 #endif
 constexpr int64_t kCacheKeepBytes = int64_t(MS_CACHE_KEEP_MIB) << 20;
 constexpr int kNormThreads = 1024;        // K2 block: 16 wave64
+static_assert(int64_t(kStatsBlocks) * kStatsBlocks <= 0x7fffffff, "K2's slot arithmetic in 32 bits");
 static_assert(kStatsBlocks % kNormThreads == 0, "K2 takes the same number of partials per thread");
 constexpr int kMaxSegs = 1 << 26;
 
@@ -1003,60 +1006,108 @@ __global__ __launch_bounds__(64 * scan_waves<kFlat>(), scan_min_waves<kFlat>()) 
 }
 
 // ------------------------------------------------------------------ K2
+// The tile statistics of a group that K2 reads itself (tiles > 0), for the
+// first kNormDirect groups of a launch; they travel in the kernel arguments.
+constexpr int kNormDirect = MS_NORM_DIRECT_GROUPS;
+struct NormTiles {
+  const double* sum[kNormDirect];
+  const uint32_t* flag[kNormDirect];
+  int32_t tiles[kNormDirect];
+};
+
+// One block.  Thread j adds a group's partial slots j, j + kNormThreads, ...,
+// waves reduce with a fixed xor tree, thread 0 adds the wave sums in order.
+// A group of at most kStatsBlocks tiles needs no fold: every slot then holds
+// one tile or none (slot j: tiles [j*T/kStatsBlocks, (j+1)*T/kStatsBlocks)),
+// and reading that tile in the slot's place gives the bits the fold would.
+// A launch of this size is all latency (K2a and K2 4.5-5 us each), so the
+// fold's launch is what there is to save.  Past kStatsBlocks tiles it stays:
+// one block reading 60,762 tiles takes 30 us against 12 for the fold and K2.
+constexpr int kNormChunk = 8;   // groups between barriers
 __global__ __launch_bounds__(kNormThreads) void k_norm_clip(
-    const double* __restrict__ bsum, const uint32_t* __restrict__ bflag,
+    const NormTiles direct, const double* __restrict__ bsum, const uint32_t* __restrict__ bflag,
     int nblk, int ngroups, int has_clip, double max_norm, int scaler_enabled,
     double scale, int64_t good_steps, int64_t skipped_steps, int64_t window,
     double min_scale, double max_scale, ms_step_scalars_t* __restrict__ out,
     ms_step_scalars_t* __restrict__ out_host) {
   constexpr int kNormWaves = kNormThreads / 64;
-  __shared__ double wsum[kNormWaves];
-  __shared__ uint32_t wbad[kNormWaves];
+  constexpr int kPer = kStatsBlocks / kNormThreads;
+  __shared__ double wsum[kNormChunk][kNormWaves];
+  __shared__ uint32_t wbad[kNormChunk][kNormWaves];
   const int tid = threadIdx.x;
   float total = 0.0f;      // meaningful in thread 0
   uint32_t overflow = 0;   // meaningful in thread 0
-  for (int gi = 0; gi < ngroups; ++gi) {
-    const double* ps = bsum + static_cast<int64_t>(gi) * nblk;
-    const uint32_t* pf = bflag + static_cast<int64_t>(gi) * nblk;
-    double acc = 0.0;
-    uint32_t bad = 0;
-    if (nblk == kStatsBlocks) {
-      // all of a thread's partials in flight at once, then added in the
-      // same order as the loop below (slot tid, tid + kNormThreads, ...)
-      constexpr int kPer = kStatsBlocks / kNormThreads;
-      double x[kPer];
-      uint32_t f[kPer];
+  for (int g0 = 0; g0 < ngroups; g0 += kNormChunk) {
+    const int g1 = g0 + kNormChunk < ngroups ? g0 + kNormChunk : ngroups;
+    for (int gi = g0; gi < g1; ++gi) {
+      const uint32_t tiles = gi < kNormDirect ? direct.tiles[gi] : 0;
+      double acc = 0.0;
+      uint32_t bad = 0;
+      // all of a thread's values in flight at once, then added in slot order
+      // (tid, tid + kNormThreads, ...)
+      if (tiles != 0) {
+        const double* ts = direct.sum[gi];
+        const uint32_t* tf = direct.flag[gi];
+        double x[kPer];
+        uint32_t f[kPer];
 #pragma unroll
-      for (int i = 0; i < kPer; ++i) {
-        x[i] = ps[tid + i * kNormThreads];
-        f[i] = pf[tid + i * kNormThreads];
-      }
+        for (int i = 0; i < kPer; ++i) {
+          const uint32_t j = static_cast<uint32_t>(tid + i * kNormThreads);
+          const uint32_t k = j * tiles / kStatsBlocks;   // < 2^28: tiles <= kStatsBlocks
+          x[i] = 0.0;
+          f[i] = 0;
+          if (k < (j + 1) * tiles / kStatsBlocks) {
+            x[i] = ts[k];
+            f[i] = tf[k];
+          }
+        }
 #pragma unroll
-      for (int i = 0; i < kPer; ++i) {
-        acc += x[i];
-        bad |= f[i];
+        for (int i = 0; i < kPer; ++i) {
+          acc += x[i];
+          bad |= f[i];
+        }
+      } else if (nblk == kStatsBlocks) {
+        const double* ps = bsum + static_cast<int64_t>(gi) * nblk;
+        const uint32_t* pf = bflag + static_cast<int64_t>(gi) * nblk;
+        double x[kPer];
+        uint32_t f[kPer];
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+          x[i] = ps[tid + i * kNormThreads];
+          f[i] = pf[tid + i * kNormThreads];
+        }
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+          acc += x[i];
+          bad |= f[i];
+        }
+      } else {
+        const double* ps = bsum + static_cast<int64_t>(gi) * nblk;
+        const uint32_t* pf = bflag + static_cast<int64_t>(gi) * nblk;
+        for (int b = tid; b < nblk; b += kNormThreads) {
+          acc += ps[b];
+          bad |= pf[b];
+        }
       }
-    } else {
-      for (int b = tid; b < nblk; b += kNormThreads) {
-        acc += ps[b];
-        bad |= pf[b];
+      const double w = wave_sum(acc);
+      const bool wb = __any(bad != 0);
+      if ((tid & 63) == 0) {
+        wsum[gi - g0][tid >> 6] = w;
+        wbad[gi - g0][tid >> 6] = wb ? 1u : 0u;
       }
-    }
-    const double w = wave_sum(acc);
-    const bool wb = __any(bad != 0);
-    if ((tid & 63) == 0) {
-      wsum[tid >> 6] = w;
-      wbad[tid >> 6] = wb ? 1u : 0u;
     }
     __syncthreads();
     if (tid == 0) {
-      double gsum = 0.0;
-      for (int k = 0; k < kNormWaves; ++k) {
-        gsum += wsum[k];
-        overflow |= wbad[k];
+      for (int gi = 0; gi < g1 - g0; ++gi) {
+        double gsum = 0.0;
+#pragma unroll
+        for (int k = 0; k < kNormWaves; ++k) {
+          gsum += wsum[gi][k];
+          overflow |= wbad[gi][k];
+        }
+        // per-group fp32 sum of squares, accumulated over groups in fp32
+        total = total + static_cast<float>(gsum);
       }
-      // per-group fp32 sum of squares, accumulated over groups in fp32
-      total = total + static_cast<float>(gsum);
     }
     __syncthreads();
   }
@@ -1583,8 +1634,13 @@ void launch_stats_s(const ms_segment_t* segs, int nseg, int64_t begin, int64_t e
                          div, flat, tsum, tflag, ntiles, 1, keep_from);
     } else {
       // runs of 2 and 4 tiles time alike over 60K-640K tiles, runs of 1 up
-      // to 30% slower
-      constexpr int kRun = MS_SCAN_RUN_READ;
+      // to 30% slower.  Up to kShortScanTiles tiles every wave gets a tile of
+      // its own in one round of the chip; runs of 4 would leave CUs idle and
+      // make each wave wait for four tiles in turn: K1 with its fold over
+      // 0.8M params in 292 segments 18.6 -> 12.2 us, 3.3M in 52 15.6 -> 11.2,
+      // 9.9M in 192 20.2 -> 16.5 (33M params, past the line: 22.7 us with
+      // runs of 1 against 21.1)
+      const int run = ntiles <= kShortScanTiles ? 1 : MS_SCAN_RUN_READ;
       // the counted elements' flags from their sums wherever the scaling
       // cannot overflow a finite gradient (GradScan's kSumFlags)
       const bool sum_flags = kScale == kScaleNone ||
@@ -1592,9 +1648,9 @@ void launch_stats_s(const ms_segment_t* segs, int nseg, int64_t begin, int64_t e
                              (kScale == kScaleDiv && div >= 1.0f);
       auto go = [&](auto sf) {
         hipLaunchKernelGGL((k_grad_stats<G, false, true, kScale, decltype(sf)::value>),
-                           dim3(scan_grid(ntiles, kScanWavesRead * kRun)),
+                           dim3(scan_grid(ntiles, kScanWavesRead * run)),
                            dim3(64 * kScanWavesRead), 0, st, segs, nseg, begin, end, ob, oe, mul,
-                           div, flat, tsum, tflag, ntiles, kRun, keep_from);
+                           div, flat, tsum, tflag, ntiles, run, keep_from);
       };
       if (sum_flags)
         go(BoolC<true>{});
@@ -1800,6 +1856,20 @@ int ms_grad_stats(const ms_segment_t* segs, int32_t nseg, int32_t grad_dtype,
                      nblk, static_cast<hipStream_t>(stream));
 }
 
+int ms_grad_tile_stats(const ms_segment_t* segs, int32_t nseg, int32_t grad_dtype,
+                       int64_t begin, int64_t end, int64_t own_begin, int64_t own_end,
+                       int32_t unscale, float grad_scale, float* flat_grad,
+                       double* tile_sumsq, uint32_t* tile_flag, int64_t ntiles, void* stream) {
+  const int rc = check_scan(segs, nseg, grad_dtype, begin, end, unscale, grad_scale);
+  if (rc != MS_OK) return rc;
+  if (!tile_sumsq || !tile_flag) return MS_EINVAL;
+  if (ntiles < scan_tiles(end - begin)) return MS_EBLOCKS;
+  if (end == begin) return MS_OK;
+  return launch_scan(segs, nseg, grad_dtype, begin, end, own_begin, own_end, unscale,
+                     grad_scale, flat_grad, tile_sumsq, tile_flag, nullptr, nullptr, 0,
+                     static_cast<hipStream_t>(stream));
+}
+
 int ms_boundary_scalars_noalloc(const ms_group_scan_t* groups, int32_t ngroups,
                                 int32_t unscale, float grad_scale, int32_t has_clip,
                                 double max_norm, int32_t scaler_enabled, double scale,
@@ -1838,8 +1908,8 @@ int ms_boundary_scalars_noalloc(const ms_group_scan_t* groups, int32_t ngroups,
                                 flags + static_cast<int64_t>(g) * kStatsBlocks, kStatsBlocks, st);
     if (lrc != MS_OK) return lrc;
   }
-  hipLaunchKernelGGL(k_norm_clip, dim3(1), dim3(kNormThreads), 0, st, sums, flags, kStatsBlocks,
-                     ngroups, has_clip, max_norm, scaler_enabled, scale, good_steps,
+  hipLaunchKernelGGL(k_norm_clip, dim3(1), dim3(kNormThreads), 0, st, NormTiles{}, sums, flags,
+                     kStatsBlocks, ngroups, has_clip, max_norm, scaler_enabled, scale, good_steps,
                      skipped_steps, window, min_scale, max_scale, out, out_host);
   return launch_status();
 }
@@ -1854,7 +1924,43 @@ int ms_norm_clip(const double* block_sumsq, const uint32_t* block_flag,
   if (nblk < kStatsBlocks) return MS_EBLOCKS;
   if (window < 1) return MS_EINVAL;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(k_norm_clip, dim3(1), dim3(kNormThreads), 0, st, block_sumsq,
+  hipLaunchKernelGGL(k_norm_clip, dim3(1), dim3(kNormThreads), 0, st, NormTiles{}, block_sumsq,
+                     block_flag, nblk, ngroups, has_clip, max_norm,
+                     scaler_enabled, scale, good_steps, skipped_steps, window,
+                     min_scale, max_scale, out, out_host);
+  return launch_status();
+}
+
+int ms_norm_clip_tiles(const ms_tile_stats_t* groups, int32_t ngroups, double* block_sumsq,
+                       uint32_t* block_flag, int32_t nblk, int32_t has_clip,
+                       double max_norm, int32_t scaler_enabled, double scale,
+                       int64_t good_steps, int64_t skipped_steps, int64_t window,
+                       double min_scale, double max_scale, ms_step_scalars_t* out,
+                       ms_step_scalars_t* out_host, void* stream) {
+  if (ngroups < 0 || (ngroups > 0 && !groups) || !block_sumsq || !block_flag || !out)
+    return MS_EINVAL;
+  if (nblk < kStatsBlocks) return MS_EBLOCKS;
+  if (window < 1) return MS_EINVAL;
+  for (int32_t g = 0; g < ngroups; ++g) {
+    const ms_tile_stats_t& ts = groups[g];
+    if (ts.ntiles < 0 || (ts.ntiles > 0 && (!ts.sumsq || !ts.flag))) return MS_EINVAL;
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  NormTiles direct = {};
+  for (int32_t g = 0; g < ngroups; ++g) {
+    const ms_tile_stats_t& ts = groups[g];
+    if (g < kNormDirect && ts.ntiles > 0 && ts.ntiles <= kStatsBlocks) {
+      direct.sum[g] = ts.sumsq;
+      direct.flag[g] = ts.flag;
+      direct.tiles[g] = static_cast<int32_t>(ts.ntiles);
+      continue;
+    }
+    launch_fold(ts.sumsq, ts.flag, ts.ntiles, block_sumsq + static_cast<int64_t>(g) * nblk,
+                block_flag + static_cast<int64_t>(g) * nblk, nblk, st);
+    const int rc = launch_status();
+    if (rc != MS_OK) return rc;
+  }
+  hipLaunchKernelGGL(k_norm_clip, dim3(1), dim3(kNormThreads), 0, st, direct, block_sumsq,
                      block_flag, nblk, ngroups, has_clip, max_norm,
                      scaler_enabled, scale, good_steps, skipped_steps, window,
                      min_scale, max_scale, out, out_host);

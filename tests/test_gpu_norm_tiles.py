@@ -1,0 +1,104 @@
+"""K2 reading the tile statistics of small groups itself
+(``ms_norm_clip_tiles``): bit for bit the fold into partial slots followed by
+``ms_norm_clip``, on both sides of the line (``ms_stats_blocks()`` tiles), for
+one group and for more groups than travel in the kernel arguments; and the
+reading K1 on both sides of its short-scan line (6144 tiles), whose tile
+slots must equal the writing K1's."""
+
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from minispeed_amd import _native
+
+DEV = "cuda:0"
+
+
+def test_arguments_refused_on_the_host():
+    lib = _native.load()
+    nb = _native.stats_blocks()
+    tail = (0, 0.0, 0, 1.0, 0, 0, 1, 1.0, 1.0)
+    groups = (_native.TileStats * 1)(_native.TileStats(None, None, 5))
+    call = lib.ms_norm_clip_tiles
+    assert call(groups, 1, 8, 8, nb, *tail, 8, None, None) == -1          # tiles without slots
+    groups[0] = _native.TileStats(8, 8, -1)
+    assert call(groups, 1, 8, 8, nb, *tail, 8, None, None) == -1
+    groups[0] = _native.TileStats(8, 8, 5)
+    assert call(None, 1, 8, 8, nb, *tail, 8, None, None) == -1
+    assert call(groups, 1, None, 8, nb, *tail, 8, None, None) == -1
+    assert call(groups, 1, 8, 8, nb, *tail, None, None, None) == -1
+    assert call(groups, 1, 8, 8, nb - 1, *tail, 8, None, None) == -3
+    assert call(groups, 1, 8, 8, nb, *tail[:6], 0, *tail[7:], 8, None, None) == -1   # window 0
+    scan = lib.ms_grad_tile_stats
+    assert scan(8, 1, 1, 0, 10, 0, 10, 0, 1.0, None, None, 8, 1, None) == -1
+    assert scan(8, 1, 1, 0, 2049, 0, 10, 0, 1.0, None, 8, 8, 1, None) == -3
+    assert scan(None, 0, 1, 0, 10, 0, 10, 0, 1.0, None, 8, 8, 1, None) == -2
+    assert scan(None, 0, 1, 4, 4, 4, 4, 0, 1.0, None, 8, 8, 0, None) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts", [[1], [63], [1024], [1025], [16383], [16384], [16385], [40000],
+                                    [0], [5, 0, 20000, 16384], [7] * 35 + [16385]])
+@pytest.mark.parametrize("bad", [None, "flag", "inf"])
+def test_norm_from_tiles_equals_fold_and_norm(counts, bad):
+    lib = _native.load()
+    nb, n = _native.stats_blocks(), len(counts)
+    gen = torch.Generator(device=DEV).manual_seed(sum(counts))
+    tiles = [(torch.rand(max(c, 1), generator=gen, device=DEV, dtype=torch.float64) * 3,
+              torch.zeros(max(c, 1), dtype=torch.int32, device=DEV)) for c in counts]
+    if bad and counts[-1]:
+        (tiles[-1][1] if bad == "flag" else tiles[-1][0])[counts[-1] - 1] = (
+            1 if bad == "flag" else float("inf"))
+    args = (1, 2.5, 1, 1024.0, 3, 1, 7, 1.0, 2.0 ** 20)
+
+    def buffers():
+        return (torch.full((n * nb,), 7.0, dtype=torch.float64, device=DEV),
+                torch.full((n * nb,), 3, dtype=torch.int32, device=DEV),
+                torch.zeros(_native.SCALARS_BYTES, dtype=torch.uint8, device=DEV))
+    ps, pf, want = buffers()
+    for g, (c, (ts, tf)) in enumerate(zip(counts, tiles)):
+        _native.check(lib.ms_reduce_tile_stats(ts.data_ptr(), tf.data_ptr(), c,
+                                               ps.data_ptr() + 8 * g * nb, pf.data_ptr() + 4 * g * nb,
+                                               nb, None), "fold")
+    _native.check(lib.ms_norm_clip(ps.data_ptr(), pf.data_ptr(), nb, n, *args, want.data_ptr(), None,
+                                   None), "norm")
+    ps, pf, got = buffers()
+    groups = (_native.TileStats * n)(*[_native.TileStats(ts.data_ptr(), tf.data_ptr(), c)
+                                       for c, (ts, tf) in zip(counts, tiles)])
+    _native.check(lib.ms_norm_clip_tiles(groups, n, ps.data_ptr(), pf.data_ptr(), nb, *args,
+                                         got.data_ptr(), None, None), "norm from tiles")
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    s = _native.StepScalars.from_buffer_copy(got.cpu().numpy().tobytes())
+    assert s.overflow == (1 if bad == "flag" and counts[-1] else 0)
+    if bad is None:
+        exact = float(np.sum([float(ts[:c].sum()) for c, (ts, _) in zip(counts, tiles)]))
+        # one fp32 rounding per group and one per add of the group sums
+        assert abs(s.sumsq - exact) <= exact * 2.0 ** -24 * 2 * n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [6144 * 2048 - 5, 6144 * 2048, 6144 * 2048 + 1])
+def test_reading_scan_equals_the_writing_scan_at_the_short_scan_line(n):
+    lib = _native.load()
+    g = torch.randn(n, device=DEV, generator=torch.Generator(device=DEV).manual_seed(1)).to(torch.float16)
+    table = torch.tensor([[0, 1000, g.data_ptr(), 0], [1000, n - 1000, g.data_ptr() + 2000, 0]],
+                         dtype=torch.int64, device=DEV)
+    nt = _native.scan_tiles(n)
+    flat = torch.empty(n, device=DEV)
+    out = []
+    for target in (None, flat.data_ptr()):
+        ts = torch.full((nt,), -1.0, dtype=torch.float64, device=DEV)
+        tf = torch.full((nt,), 9, dtype=torch.int32, device=DEV)
+        _native.check(lib.ms_grad_tile_stats(table.data_ptr(), 2, _native.DTYPE_F16, 0, n, 0, n,
+                                             _native.SCALE_DIVIDE, 1024.0, target, ts.data_ptr(),
+                                             tf.data_ptr(), nt, None), "K1")
+        out.append((ts, tf))
+    torch.cuda.synchronize()
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    assert torch.equal(flat, g.float() / 1024.0)
+    assert int(out[0][1].max()) == 0
