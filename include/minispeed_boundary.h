@@ -228,6 +228,19 @@ int ms_grad_tile_stats(const ms_segment_t* segs, int32_t nseg, int32_t grad_dtyp
                        double* tile_sumsq, uint32_t* tile_flag, int64_t ntiles,
                        void* stream);
 
+/* K1 over one contiguous buffer of n elements of `dtype` [dev], with no
+ * segment table: the tile slots ms_grad_tile_stats writes for a one-row
+ * table that counts every element, without scaling (has_overflow,
+ * precision.py:79-87; local_grad_sumsq, flat.py:232-234). */
+int ms_buffer_tile_stats(const void* buf, int32_t dtype, int64_t n, double* tile_sumsq,
+                         uint32_t* tile_flag, int64_t ntiles, void* stream);
+
+/* buf[i] /= factor (MS_SCALE_DIVIDE, factor > 0; unscale_grads,
+ * flat.py:243-247) or buf[i] *= factor (MS_SCALE_MULTIPLY; scale_grads,
+ * flat.py:249-257) for i in [0, n), as ms_grad_stats scales in place
+ * (MS_SCALE_NONE: nothing). */
+int ms_buffer_scale(float* buf, int64_t n, int32_t mode, float factor, void* stream);
+
 /* The tile statistics of one group: ntiles slots [dev] that K1
  * (ms_grad_tile_stats) or K5 (ms_accumulate_grads) wrote.  The pointers may
  * be NULL when ntiles is 0 (a group that adds nothing). */

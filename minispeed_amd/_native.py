@@ -155,6 +155,8 @@ SIGNATURES = {
         ctypes.c_int,
         [_P, _I32, _I32, _I64, _I64, _I64, _I64, _I32, _F, _P, _P, _P, _I64, _P],
     ),
+    "ms_buffer_tile_stats": (ctypes.c_int, [_P, _I32, _I64, _P, _P, _I64, _P]),
+    "ms_buffer_scale": (ctypes.c_int, [_P, _I64, _I32, _F, _P]),
     "ms_norm_clip_tiles": (
         ctypes.c_int,
         [ctypes.POINTER(TileStats), _I32, _P, _P, _I32, _I32, _D, _I32, _D, _I64, _I64, _I64, _D, _D,

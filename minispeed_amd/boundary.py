@@ -135,15 +135,7 @@ class Workspace:
         # polls (HostReadback): no copy, and K3, queued behind K2, keeps
         # running while the host does its bookkeeping
         self.readback = HostReadback()
-        self.host = self.readback.host
         self._stream: Optional[torch.cuda.Stream] = None   # stream of the last boundary
-
-    def partial_ptrs(self, g: int):
-        off = g * self.nblk
-        return (
-            self.partials.data_ptr() + off * 8,
-            self.flags.data_ptr() + off * 4,
-        )
 
     def tile_ptrs(self, ntiles: int):
         """Addresses (sums, flags) of at least ``ntiles`` K1 tile slots for
@@ -160,12 +152,6 @@ class Workspace:
             self.tile_flags.record_stream(cur)
             self._tile_streams.add(cur.cuda_stream)
         return self.tile_sums.data_ptr(), self.tile_flags.data_ptr()
-
-    def read_scalars(self) -> _native.StepScalars:
-        """Copy K2's result to pinned memory and wait for the stream."""
-        self.host.copy_(self.scalars, non_blocking=True)
-        torch.cuda.current_stream(self.device).synchronize()
-        return _native.StepScalars.from_buffer_copy(self.host.numpy().tobytes())
 
     def enter(self) -> torch.cuda.Stream:
         """Called at the start of a boundary; returns the current stream,
@@ -405,12 +391,6 @@ def run_boundary(
 
 
 # ------------------------------------------------------------------ utility
-def _whole_buffer_table(flat: torch.Tensor) -> torch.Tensor:
-    """Device segment table of one row covering a contiguous buffer."""
-    table = np.array([[0, flat.numel(), flat.data_ptr(), 0]], dtype=np.int64)
-    return torch.from_numpy(table).to(flat.device)
-
-
 def scale_in_place(buf: torch.Tensor, mode: int, factor: float) -> None:
     """``buf.div_(factor)`` (mode SCALE_DIVIDE, flat.py:243-247) or
     ``buf.mul_(factor)`` (mode SCALE_MULTIPLY, flat.py:249-257) of a
@@ -419,62 +399,80 @@ def scale_in_place(buf: torch.Tensor, mode: int, factor: float) -> None:
     _native.require_hip_tensor(buf, "scaled buffer")
     if buf.dtype != torch.float32 or not buf.is_contiguous():
         raise TypeError("scale_in_place needs a contiguous float32 buffer")
-    n = buf.numel()
-    if n == 0:
+    if buf.numel() == 0:
         return
-    table = _whole_buffer_table(buf)
-    _native.check(_native.load().ms_grad_stats(
-        table.data_ptr(), 1, _native.DTYPE_F32, 0, n, 0, 0, mode, float(np.float32(factor)),
-        buf.data_ptr(), None, None, 0, None, None, 0, _native.stream_handle(buf.device)),
-        "ms_grad_stats(scale)")
+    _native.check(_native.load().ms_buffer_scale(
+        buf.data_ptr(), buf.numel(), mode, float(np.float32(factor)),
+        _native.stream_handle(buf.device)), "ms_buffer_scale")
+
+
+def _scan_buffers(bufs: Sequence[torch.Tensor], readback: Optional[HostReadback] = None) -> torch.Tensor:
+    """K1 over each buffer, then K2 over all of them (in order, one group
+    each): the ``ms_step_scalars_t`` as device bytes, and through
+    ``readback`` on the host.  The scratch is one allocation on the current
+    stream, which orders its reuse after the kernels."""
+    lib = _native.load()
+    device = bufs[0].device
+    stream = _native.stream_handle(device)
+    nblk = _native.stats_blocks()
+    tiles = [_native.scan_tiles(b.numel()) for b in bufs]
+    n, slots = len(bufs), len(bufs) * nblk + sum(tiles)
+    scratch = torch.empty(12 * slots, dtype=torch.uint8, device=device)
+    scalars = torch.empty(_native.SCALARS_BYTES, dtype=torch.uint8, device=device)
+    sums = scratch.data_ptr()                 # fp64 slots, then the uint32 ones
+    flags = sums + 8 * slots
+    stats = (_native.TileStats * n)()
+    tsum, tflag = sums + 8 * n * nblk, flags + 4 * n * nblk
+    for st, b, nt in zip(stats, bufs, tiles):
+        _native.check(lib.ms_buffer_tile_stats(b.data_ptr(), _native.ms_dtype(b.dtype), b.numel(),
+                                               tsum, tflag, nt, stream), "ms_buffer_tile_stats")
+        st.sumsq, st.flag, st.ntiles = tsum, tflag, nt
+        tsum += 8 * nt
+        tflag += 4 * nt
+    if readback is not None:
+        readback.arm()
+    _native.check(lib.ms_norm_clip_tiles(stats, n, sums, flags, nblk, 0, 0.0, 0, 1.0, 0, 0, 1, 1.0,
+                                         1.0, scalars.data_ptr(),
+                                         None if readback is None else readback.ptr, stream),
+                  "ms_norm_clip_tiles")
+    return scalars
+
+
+def _scan_to_host(bufs: Sequence[torch.Tensor]) -> _native.StepScalars:
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("a scan whose result the host waits for cannot run under graph capture")
+    readback = HostReadback()
+    _scan_buffers(bufs, readback)
+    return readback.wait(_native.stream_handle(bufs[0].device))
+
+
+def _flat_view(buf: torch.Tensor) -> torch.Tensor:
+    return buf.detach().reshape(-1).contiguous()
 
 
 def sumsq_device(buf: torch.Tensor) -> torch.Tensor:
     """``buf.pow(2).sum()`` as a 0-dim fp32 device tensor (flat.py:232-234):
-    K1's fp64 tile partials, folded into K2's slots, summed by K2 and rounded
-    to fp32 once."""
+    K1's fp64 tile partials, summed by K2 and rounded to fp32 once."""
     _native.require_hip_tensor(buf, "sum-of-squares buffer")
-    flat = buf.detach().reshape(-1)
-    if not flat.is_contiguous():
-        flat = flat.contiguous()
-    n = flat.numel()
-    if n == 0:
-        return torch.zeros((), dtype=torch.float32, device=flat.device)
-    lib = _native.load()
-    ws = Workspace(flat.device, 1)
-    table = _whole_buffer_table(flat)
-    stream = _native.stream_handle(flat.device)
-    psum, pflag = ws.partial_ptrs(0)
-    ntiles = _native.scan_tiles(n)
-    tsum, tflag = ws.tile_ptrs(ntiles)
-    _native.check(lib.ms_grad_stats(table.data_ptr(), 1, _native.ms_dtype(flat.dtype), 0, n, 0, n, 0,
-                                    1.0, None, tsum, tflag, ntiles, psum, pflag, ws.nblk, stream),
-                  "ms_grad_stats")
-    _native.check(lib.ms_norm_clip(psum, pflag, ws.nblk, 1, 0, 0.0, 0, 1.0, 0, 0, 1, 1.0, 1.0,
-                                   ws.scalars.data_ptr(), None, stream), "ms_norm_clip")
+    if buf.numel() == 0:
+        return torch.zeros((), dtype=torch.float32, device=buf.device)
+    scalars = _scan_buffers([_flat_view(buf)])
     off = _native.StepScalars.sumsq.offset
-    return ws.scalars[off:off + 4].view(torch.float32).clone().reshape(())
+    return scalars[off:off + 4].view(torch.float32).reshape(())
+
+
+def norm_of(bufs: Sequence[torch.Tensor]) -> float:
+    """The global L2 norm of the buffers (stage_1_and_2.py:114-121): every
+    buffer's sum of squares as :func:`sumsq_device` gives it, added in order
+    in fp32, fp32 square root; one wait for the host's copy."""
+    for buf in bufs:
+        _native.require_hip_tensor(buf, "sum-of-squares buffer")
+    return float(_scan_to_host([_flat_view(b) for b in bufs]).norm)
 
 
 def scan_nonfinite(buf: torch.Tensor) -> bool:
     """inf/nan test of one device buffer with K1 + K2 (used by
     precision.has_overflow)."""
     _native.require_hip_tensor(buf, "has_overflow buffer")
-    flat = buf.detach().reshape(-1)
-    if not flat.is_contiguous():
-        flat = flat.contiguous()
-    n = flat.numel()
-    dtype = _native.ms_dtype(flat.dtype)
-    lib = _native.load()
-    ws = Workspace(flat.device, 1)
-    dev_table = _whole_buffer_table(flat)
-    stream = _native.stream_handle(flat.device)
-    psum, pflag = ws.partial_ptrs(0)
-    ntiles = _native.scan_tiles(n)
-    tsum, tflag = ws.tile_ptrs(ntiles)
-    _native.check(lib.ms_grad_stats(dev_table.data_ptr(), 1, dtype, 0, n, 0, 0, 0, 1.0,
-                                    None, tsum, tflag, ntiles, psum, pflag, ws.nblk, stream),
-                  "ms_grad_stats")
-    _native.check(lib.ms_norm_clip(psum, pflag, ws.nblk, 1, 0, 0.0, 0, 1.0, 0, 0, 1, 1.0, 1.0,
-                                   ws.scalars.data_ptr(), None, stream), "ms_norm_clip")
-    return bool(ws.read_scalars().overflow)
+    _native.ms_dtype(buf.dtype)
+    return bool(_scan_to_host([_flat_view(buf)]).overflow)

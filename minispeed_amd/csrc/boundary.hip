@@ -829,12 +829,24 @@ __device__ void scan_tile(Scan& sc, const ms_segment_t* segs, int nseg, int& s, 
 // inside a unit of its storage is split the same way with its head and
 // tail elements (split_tile_shifted).  Any other tile is scanned by wave 0
 // alone, as when reading.
-template <class G, bool kFlat, bool kStats, int kScale, bool kSumFlags = false>
+//
+// kOne: the table is the one row `one` of the kernel arguments (nseg is 1): a
+// scan of one contiguous buffer then needs no table in device memory, whose
+// upload from the host waits for the stream and left 35-40 us before each
+// such scan.  The row is read where it lies, at the start of the kernel
+// argument segment: with its fields in registers the compiler folds the walk
+// away, hoists its branches and spills 80-94 registers.
+template <class G, bool kFlat, bool kStats, int kScale, bool kSumFlags = false, bool kOne = false>
 __global__ __launch_bounds__(64 * scan_waves<kFlat>(), scan_min_waves<kFlat>()) void k_grad_stats(
-    const ms_segment_t* __restrict__ segs, int nseg, int64_t begin,
+    const ms_segment_t one, const ms_segment_t* __restrict__ table, int nseg, int64_t begin,
     int64_t end, int64_t own_begin, int64_t own_end, float mul, float div,
     float* __restrict__ flat, double* __restrict__ tsum, uint32_t* __restrict__ tflag,
     int64_t ntiles, int run, int64_t keep_from) {
+  const ms_segment_t* segs;
+  if constexpr (kOne)
+    segs = (const ms_segment_t*)(const void*)__builtin_amdgcn_kernarg_segment_ptr();
+  else
+    segs = table;
   static_assert(!(kFlat && kSumFlags), "writing, the flags come from the per-word tests");
   constexpr int kWaves = scan_waves<kFlat>();
   using Scan = GradScan<G, kFlat, kStats, kScale>;
@@ -1620,27 +1632,54 @@ int scan_grid(int64_t ntiles, int tiles_per_block) {
   return static_cast<int>(g);
 }
 
+// Tiles per wave of the reading K1.  Runs of 2 and 4 tiles time alike over
+// 60K-640K tiles, runs of 1 up to 30% slower.  Up to kShortScanTiles tiles
+// every wave gets a tile of its own in one round of the chip; runs of 4 would
+// leave CUs idle and make each wave wait for four tiles in turn: K1 with its
+// fold over 0.8M params in 292 segments 18.6 -> 12.2 us, 3.3M in 52 15.6 ->
+// 11.2, 9.9M in 192 20.2 -> 16.5 (33M params, past the line: 22.7 us with
+// runs of 1 against 21.1).
+int scan_run_tiles(int64_t ntiles) { return ntiles <= kShortScanTiles ? 1 : MS_SCAN_RUN_READ; }
+
+// the first of the tiles holding the last kCacheKeepBytes of gradient
+template <class G>
+int64_t keep_from_tile(int64_t ntiles) {
+  const int64_t keep = kCacheKeepBytes / (int64_t(kScanTile) * G::kBytes);
+  return ntiles > keep ? ntiles - keep : 0;
+}
+
+// K1 over one contiguous buffer (kOne): its statistics, or scaled in place
+template <class G>
+void launch_buffer_stats(const ms_segment_t& one, double* tsum, uint32_t* tflag, hipStream_t st) {
+  const int64_t n = one.numel, ntiles = scan_tiles(n);
+  const int run = scan_run_tiles(ntiles);
+  hipLaunchKernelGGL((k_grad_stats<G, false, true, kScaleNone, true, true>),
+                     dim3(scan_grid(ntiles, kScanWavesRead * run)), dim3(64 * kScanWavesRead), 0,
+                     st, one, nullptr, 1, 0, n, 0, n, 1.0f, 1.0f, nullptr, tsum, tflag, ntiles, run,
+                     keep_from_tile<G>(ntiles));
+}
+
+template <int kScale>
+void launch_buffer_scale(const ms_segment_t& one, float mul, float div, hipStream_t st) {
+  const int64_t n = one.numel, ntiles = scan_tiles(n);
+  hipLaunchKernelGGL((k_grad_stats<DF32, true, false, kScale, false, true>),
+                     dim3(scan_grid(ntiles, 1)), dim3(64 * kScanWavesFlat), 0, st, one, nullptr, 1, 0, n,
+                     0, 0, mul, div, static_cast<float*>(const_cast<void*>(one.grad)), nullptr,
+                     nullptr, ntiles, 1, ntiles);
+}
+
 template <class G, int kScale>
 void launch_stats_s(const ms_segment_t* segs, int nseg, int64_t begin, int64_t end, int64_t ob,
                     int64_t oe, float mul, float div, float* flat, double* tsum, uint32_t* tflag,
                     int64_t ntiles, hipStream_t st) {
-  // the tiles holding the last kCacheKeepBytes of gradient
-  const int64_t keep_tiles = kCacheKeepBytes / (int64_t(kScanTile) * G::kBytes);
-  const int64_t keep_from = ntiles > keep_tiles ? ntiles - keep_tiles : 0;
+  const int64_t keep_from = keep_from_tile<G>(ntiles);
   if (tsum) {
     if (flat) {
       hipLaunchKernelGGL((k_grad_stats<G, true, true, kScale>), dim3(scan_grid(ntiles, 1)),
-                         dim3(64 * kScanWavesFlat), 0, st, segs, nseg, begin, end, ob, oe, mul,
-                         div, flat, tsum, tflag, ntiles, 1, keep_from);
+                         dim3(64 * kScanWavesFlat), 0, st, ms_segment_t{}, segs, nseg, begin, end,
+                         ob, oe, mul, div, flat, tsum, tflag, ntiles, 1, keep_from);
     } else {
-      // runs of 2 and 4 tiles time alike over 60K-640K tiles, runs of 1 up
-      // to 30% slower.  Up to kShortScanTiles tiles every wave gets a tile of
-      // its own in one round of the chip; runs of 4 would leave CUs idle and
-      // make each wave wait for four tiles in turn: K1 with its fold over
-      // 0.8M params in 292 segments 18.6 -> 12.2 us, 3.3M in 52 15.6 -> 11.2,
-      // 9.9M in 192 20.2 -> 16.5 (33M params, past the line: 22.7 us with
-      // runs of 1 against 21.1)
-      const int run = ntiles <= kShortScanTiles ? 1 : MS_SCAN_RUN_READ;
+      const int run = scan_run_tiles(ntiles);
       // the counted elements' flags from their sums wherever the scaling
       // cannot overflow a finite gradient (GradScan's kSumFlags)
       const bool sum_flags = kScale == kScaleNone ||
@@ -1649,8 +1688,8 @@ void launch_stats_s(const ms_segment_t* segs, int nseg, int64_t begin, int64_t e
       auto go = [&](auto sf) {
         hipLaunchKernelGGL((k_grad_stats<G, false, true, kScale, decltype(sf)::value>),
                            dim3(scan_grid(ntiles, kScanWavesRead * run)),
-                           dim3(64 * kScanWavesRead), 0, st, segs, nseg, begin, end, ob, oe, mul,
-                           div, flat, tsum, tflag, ntiles, run, keep_from);
+                           dim3(64 * kScanWavesRead), 0, st, ms_segment_t{}, segs, nseg, begin, end,
+                           ob, oe, mul, div, flat, tsum, tflag, ntiles, run, keep_from);
       };
       if (sum_flags)
         go(BoolC<true>{});
@@ -1659,8 +1698,8 @@ void launch_stats_s(const ms_segment_t* segs, int nseg, int64_t begin, int64_t e
     }
   } else {
     hipLaunchKernelGGL((k_grad_stats<G, true, false, kScale>), dim3(scan_grid(ntiles, 1)),
-                       dim3(64 * kScanWavesFlat), 0, st, segs, nseg, begin, end, ob, oe, mul, div,
-                       flat, tsum, tflag, ntiles, 1, ntiles);
+                       dim3(64 * kScanWavesFlat), 0, st, ms_segment_t{}, segs, nseg, begin, end, ob,
+                       oe, mul, div, flat, tsum, tflag, ntiles, 1, ntiles);
   }
 }
 
@@ -1868,6 +1907,51 @@ int ms_grad_tile_stats(const ms_segment_t* segs, int32_t nseg, int32_t grad_dtyp
   return launch_scan(segs, nseg, grad_dtype, begin, end, own_begin, own_end, unscale,
                      grad_scale, flat_grad, tile_sumsq, tile_flag, nullptr, nullptr, 0,
                      static_cast<hipStream_t>(stream));
+}
+
+int ms_buffer_tile_stats(const void* buf, int32_t dtype, int64_t n, double* tile_sumsq,
+                         uint32_t* tile_flag, int64_t ntiles, void* stream) {
+  if (!valid_dtype(dtype) || n < 0 || (n > 0 && !buf) || !tile_sumsq || !tile_flag)
+    return MS_EINVAL;
+  if (ntiles < scan_tiles(n)) return MS_EBLOCKS;
+  if (n == 0) return MS_OK;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const ms_segment_t one{0, n, buf, nullptr};
+  switch (dtype) {
+    case MS_DTYPE_F32:
+      launch_buffer_stats<DF32>(one, tile_sumsq, tile_flag, st);
+      break;
+    case MS_DTYPE_F16:
+      launch_buffer_stats<DF16>(one, tile_sumsq, tile_flag, st);
+      break;
+    default:
+      launch_buffer_stats<DBF16>(one, tile_sumsq, tile_flag, st);
+      break;
+  }
+  return launch_status();
+}
+
+int ms_buffer_scale(float* buf, int64_t n, int32_t mode, float factor, void* stream) {
+  if (n < 0 || (n > 0 && !buf)) return MS_EINVAL;
+  if (mode != MS_SCALE_NONE && mode != MS_SCALE_DIVIDE && mode != MS_SCALE_MULTIPLY)
+    return MS_EINVAL;
+  if (mode == MS_SCALE_DIVIDE && !(factor > 0.0f)) return MS_EINVAL;
+  if (n == 0 || mode == MS_SCALE_NONE) return MS_OK;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const ms_segment_t one{0, n, buf, nullptr};
+  float inv = 1.0f;
+  switch (unscale_mode(mode, factor, &inv)) {
+    case 1:   // x / 2^k as x * 2^-k
+      launch_buffer_scale<kScaleMul>(one, inv, 1.0f, st);
+      break;
+    case 3:
+      launch_buffer_scale<kScaleMul>(one, factor, 1.0f, st);
+      break;
+    default:
+      launch_buffer_scale<kScaleDiv>(one, 1.0f, factor, st);
+      break;
+  }
+  return launch_status();
 }
 
 int ms_boundary_scalars_noalloc(const ms_group_scan_t* groups, int32_t ngroups,

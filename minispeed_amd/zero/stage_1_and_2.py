@@ -17,7 +17,7 @@ from typing import List, Optional
 import torch
 
 from .. import _native, comm
-from ..boundary import GroupLaunch, LaunchTimer, Workspace, run_boundary
+from ..boundary import GroupLaunch, LaunchTimer, Workspace, norm_of, run_boundary
 from ..flat import FlatParamGroup
 from ..optim.adam import FlatAdam
 
@@ -88,10 +88,7 @@ class ZeROOptimizer:
         gradients (group sums of squares added in fp32, fp32 sqrt), and, if
         ``max_norm`` is set and the norm exceeds it, every group's owned
         gradients multiplied by ``max_norm / (norm + 1e-6)``."""
-        total = torch.zeros((), dtype=torch.float32, device=self.flat_groups[0].device)
-        for g in self.flat_groups:
-            total += g.local_grad_sumsq()
-        norm = float(total.sqrt().item())
+        norm = norm_of([g.grad_for_shard() for g in self.flat_groups])
         self.grad_norm = norm
         if max_norm is not None and norm > max_norm:
             coef = max_norm / (norm + 1e-6)

@@ -3,7 +3,9 @@
 ``ms_norm_clip``, on both sides of the line (``ms_stats_blocks()`` tiles), for
 one group and for more groups than travel in the kernel arguments; and the
 reading K1 on both sides of its short-scan line (6144 tiles), whose tile
-slots must equal the writing K1's."""
+slots must equal the writing K1's; and K1 over one contiguous buffer without a
+segment table (``ms_buffer_tile_stats``, ``ms_buffer_scale``), bit for bit the
+scan of a one-row table, torch's ``div_`` and ``mul_``."""
 
 from __future__ import annotations
 
@@ -38,6 +40,13 @@ def test_arguments_refused_on_the_host():
     assert scan(8, 1, 1, 0, 2049, 0, 10, 0, 1.0, None, 8, 8, 1, None) == -3
     assert scan(None, 0, 1, 0, 10, 0, 10, 0, 1.0, None, 8, 8, 1, None) == -2
     assert scan(None, 0, 1, 4, 4, 4, 4, 0, 1.0, None, 8, 8, 0, None) == 0
+    stats, scale = lib.ms_buffer_tile_stats, lib.ms_buffer_scale
+    assert stats(8, 7, 10, 8, 8, 1, None) == -1 and stats(8, 0, -1, 8, 8, 1, None) == -1
+    assert stats(None, 0, 10, 8, 8, 1, None) == -1 and stats(8, 0, 10, 8, None, 1, None) == -1
+    assert stats(8, 0, 2049, 8, 8, 1, None) == -3 and stats(None, 0, 0, 8, 8, 0, None) == 0
+    assert scale(None, 10, 1, 2.0, None) == -1 and scale(8, -1, 1, 2.0, None) == -1
+    assert scale(8, 10, 3, 2.0, None) == -1 and scale(8, 10, 1, 0.0, None) == -1
+    assert scale(None, 0, 2, 0.0, None) == 0 and scale(8, 10, 0, 2.0, None) == 0
 
 
 @pytest.mark.gpu
@@ -102,3 +111,44 @@ def test_reading_scan_equals_the_writing_scan_at_the_short_scan_line(n):
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
     assert torch.equal(flat, g.float() / 1024.0)
     assert int(out[0][1].max()) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 7, 2047, 2048, 2049, 3 * 2048 + 5, 6200 * 2048 + 1])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("off", [0, 1])
+def test_buffer_scan_equals_the_one_row_table(n, dtype, off):
+    lib = _native.load()
+    gen = torch.Generator(device=DEV).manual_seed(n + off)
+    x = torch.randn(n + off, generator=gen, device=DEV).to(dtype)[off:]
+    if n > 1:
+        x[n // 2] = float("nan" if n % 2 else "inf")
+    nt = _native.scan_tiles(n)
+    table = torch.tensor([[0, n, x.data_ptr(), 0]], dtype=torch.int64, device=DEV)
+    out = []
+    for one in (True, False):
+        ts = torch.full((nt,), -1.0, dtype=torch.float64, device=DEV)
+        tf = torch.full((nt,), 9, dtype=torch.int32, device=DEV)
+        args = (ts.data_ptr(), tf.data_ptr(), nt, None)
+        d = _native.ms_dtype(dtype)
+        rc = (lib.ms_buffer_tile_stats(x.data_ptr(), d, n, *args) if one else
+              lib.ms_grad_tile_stats(table.data_ptr(), 1, d, 0, n, 0, n, 0, 1.0, None, *args))
+        _native.check(rc, "K1")
+        out.append((ts, tf))
+    torch.cuda.synchronize()
+    assert torch.equal(out[0][0].view(torch.int64), out[1][0].view(torch.int64))
+    assert torch.equal(out[0][1], out[1][1])
+    assert int(out[0][1].sum()) == (1 if n > 1 else 0)
+    if dtype is not torch.float32:
+        return
+    for mode, factor in ((_native.SCALE_DIVIDE, 1024.0), (_native.SCALE_DIVIDE, 3.0),
+                         (_native.SCALE_MULTIPLY, 1.0 / 3.0)):
+        want = x.cpu()
+        want.div_(factor) if mode == _native.SCALE_DIVIDE else want.mul_(factor)
+        y = torch.cat([torch.full((8 + off,), 5.0, device=DEV), x, torch.full((8,), 5.0, device=DEV)])
+        inner = y[8 + off:8 + off + n]
+        _native.check(lib.ms_buffer_scale(inner.data_ptr(), n, mode, float(np.float32(factor)), None),
+                      "scale")
+        torch.cuda.synchronize()
+        assert torch.equal(torch.nan_to_num(inner.cpu()), torch.nan_to_num(want))
+        assert bool((y[:8 + off] == 5.0).all()) and bool((y[8 + off + n:] == 5.0).all())
