@@ -56,7 +56,7 @@ import numpy as np
 import torch
 
 from . import _native
-from .flat import FlatParamGroup, record_streams
+from .flat import FlatParamGroup, _walk, record_streams
 
 
 # K5's row layout (ms_accum_row_t) as a numpy record
@@ -77,7 +77,11 @@ def accumulate_rows(rows: np.ndarray, src_dtype: int, device: torch.device,
     ``scale`` (``unscale``: SCALE_NONE or SCALE_DIVIDE) for them."""
     if len(rows) == 0:
         return
-    rows = np.ascontiguousarray(rows, dtype=ACCUM_ROW)
+    _launch_rows(np.ascontiguousarray(rows, dtype=ACCUM_ROW), src_dtype, device, unscale, scale)
+
+
+def _launch_rows(rows: np.ndarray, src_dtype: int, device: torch.device, unscale: int,
+                 scale: float) -> None:
     rc = _native.load().ms_accumulate_grads(rows.ctypes.data, len(rows), src_dtype, unscale,
                                             ctypes.c_float(scale).value,
                                             _native.stream_handle(device))
@@ -95,7 +99,6 @@ class ContiguousGradients:
     def __init__(self, groups: List[FlatParamGroup], bucket_elements: int = BUCKET_ELEMENTS,
                  scale_fn: Optional[Callable[[], float]] = None):
         self.groups = groups
-        self.window = 0
         self.bucket_elements = int(bucket_elements)
         # the loss scale the boundary will unscale by (the engine's scaler)
         self.scale_fn = scale_fn or (lambda: 1.0)
@@ -103,29 +106,27 @@ class ContiguousGradients:
         self.use_tile_stats = True
         self.accum = [torch.empty(g.numel_padded, dtype=torch.float32, device=g.device)
                       for g in groups]
-        self._offsets = [np.asarray(g.layout.offsets, dtype=np.int64) for g in groups]
         # statistics slots: parameter k of group g owns ceil(numel / 2048)
-        # tiles from _tile0[g][k]
+        # tiles; the queued gradients, not yet added, in hook order
         tile = _native.ACCUM_TILE
-        self._tile0, self.tile_sumsq, self.tile_flag = [], [], []
-        for g in groups:
+        self.tile_sumsq, self.tile_flag = [], []
+        self._queue = _walk().GradQueue()
+        for g, accum in zip(groups, self.accum):
             counts = (np.asarray(g._numels, dtype=np.int64) + tile - 1) // tile
-            self._tile0.append(np.concatenate([[0], np.cumsum(counts)[:-1]]).astype(np.int64))
+            tile0 = np.concatenate([[0], np.cumsum(counts)[:-1]]).astype(np.int64)
             n = int(counts.sum())
             self.tile_sumsq.append(torch.zeros(n, dtype=torch.float64, device=g.device))
             self.tile_flag.append(torch.zeros(n, dtype=torch.int32, device=g.device))
+            self._queue.add_group(g._device_index, list(g._numels), list(g.layout.offsets),
+                                  tile0.tolist(), accum.data_ptr(),
+                                  self.tile_sumsq[-1].data_ptr(), self.tile_flag[-1].data_ptr())
+        self._take, self._slow = self._queue.take, self._queue.SLOW
         # the (unscale, fp32 scale) of this window's flushes; None before the
         # first, False once two differed
         self._window_unscale = None
         # the stream of the last boundary (the sums and slots were read and
         # cleared there): a flush on another stream waits for it first
         self._boundary_stream: Optional[torch.cuda.Stream] = None
-        # window in which each parameter last contributed (-1: never)
-        self._seen = [np.full(len(g.params), -1, dtype=np.int64) for g in groups]
-        # queued (group, index, gradient, first) in hook order, not yet added
-        self._queue: List[Tuple[int, int, torch.Tensor, bool]] = []
-        self._queued = set()
-        self._queued_numel = 0
         self._callback_pending = False
         self._handles = []
         for gi, g in enumerate(groups):
@@ -146,13 +147,23 @@ class ContiguousGradients:
         self._callback_pending = False
         self.flush()
 
-    @torch.no_grad()
     def accumulate(self, gi: int, k: int, param: torch.nn.Parameter) -> None:
         """Queue ``param.grad`` for its fp32 slice and release it (K5 adds it
         at the next :meth:`flush`)."""
+        queued = self._take(gi, k, param)
+        if queued <= self._slow:
+            queued = self._accumulate_checked(gi, k, param)
+        if queued >= self.bucket_elements:
+            self.flush()
+
+    @torch.no_grad()
+    def _accumulate_checked(self, gi: int, k: int, param: torch.nn.Parameter) -> int:
+        """A gradient the queue does not take by itself: refused here with
+        the precise error, made contiguous, or preceded by a flush of the
+        parameter's earlier one."""
         grad = param.grad
         if grad is None:
-            return
+            return self._queue.NONE
         g = self.groups[gi]
         n = g._numels[k]
         if grad.numel() != n:
@@ -161,61 +172,44 @@ class ContiguousGradients:
         if grad.device != g.device:
             raise RuntimeError(f"gradient on {grad.device}, expected {g.device}")
         _native.ms_dtype(grad.dtype)        # f32 / f16 / bf16 only
-        if (gi, k) in self._queued:
+        grad = grad.contiguous()
+        queued = self._queue.put(gi, k, grad)
+        if queued == self._queue.AGAIN:
             self.flush()                    # its earlier gradient goes first
-        self._queue.append((gi, k, grad.contiguous(), self._seen[gi][k] != self.window))
-        self._queued.add((gi, k))
-        self._queued_numel += n
-        self._seen[gi][k] = self.window
+            queued = self._queue.put(gi, k, grad)
         param.grad = None
-        if self._queued_numel >= self.bucket_elements:
-            self.flush()
+        return queued
 
     @torch.no_grad()
     def flush(self) -> None:
         """Add every queued gradient into its slice, with its tiles'
         statistics: one batched K5 call per (device, gradient dtype), then
         drop the gradients."""
-        if not self._queue:
+        if self._queue.empty():
             return
-        queue, self._queue = self._queue, []
-        self._queued.clear()
-        self._queued_numel = 0
+        batches = self._queue.rows()
         unscale = unscale_of(float(self.scale_fn()))
         if self._window_unscale is None:
             self._window_unscale = unscale
         elif self._window_unscale != unscale:
             self._window_unscale = False
-        batches = {}
-        for gi, k, grad, first in queue:
-            batches.setdefault((self.groups[gi].device, grad.dtype), []).append((gi, k, grad, first))
-        for (device, dtype), items in batches.items():
+        for index, dtype, rows, grads in batches:
+            device = torch.device("cuda", index)
             cur = torch.cuda.current_stream(device)
             prev = self._boundary_stream
             if prev is not None and prev.device == device and prev != cur:
                 cur.wait_stream(prev)
-            rows = np.zeros(len(items), dtype=ACCUM_ROW)
-            rows["dst"] = [self.accum[gi].data_ptr() + int(self._offsets[gi][k]) * 4
-                           for gi, k, _, _ in items]
-            rows["src"] = [grad.data_ptr() for _, _, grad, _ in items]
-            rows["numel"] = [grad.numel() for _, _, grad, _ in items]
-            rows["first"] = [1 if first else 0 for _, _, _, first in items]
-            rows["tile_sumsq"] = [self.tile_sumsq[gi].data_ptr() + int(self._tile0[gi][k]) * 8
-                                  for gi, k, _, _ in items]
-            rows["tile_flag"] = [self.tile_flag[gi].data_ptr() + int(self._tile0[gi][k]) * 4
-                                 for gi, k, _, _ in items]
-            accumulate_rows(rows, _native.ms_dtype(dtype), device, unscale[0], unscale[1])
+            _launch_rows(rows, dtype, device, *unscale)
             # the gradients' memory goes back to the caching allocator, which
             # hands it out again only in the order of this stream
-            record_streams([grad for _, _, grad, _ in items], cur)
+            record_streams(grads, cur)
 
     def grad_pointers(self, gi: int) -> np.ndarray:
         """Addresses of the fp32 sums of group ``gi`` (0 for parameters
         without a gradient this window), with the padding row's trailing 0."""
         self.flush()
-        seen = self._seen[gi] == self.window
         ptrs = np.zeros(len(self.groups[gi].params) + 1, dtype=np.int64)
-        ptrs[:-1] = np.where(seen, self.accum[gi].data_ptr() + self._offsets[gi] * 4, 0)
+        self._queue.pointers(gi, ptrs)
         return ptrs
 
     def tile_stats(self, gi: int, scale: float) -> Optional[Tuple[int, int, int]]:
@@ -236,9 +230,7 @@ class ContiguousGradients:
         """Forget the sums (the boundary consumed them, or zero_grad): the
         statistics slots are cleared on the current stream; queued
         gradients of the abandoned window are dropped unread."""
-        self._queue = []
-        self._queued.clear()
-        self._queued_numel = 0
+        self._queue.next_window()
         self._callback_pending = False
         self._window_unscale = None
         for ts, tf in zip(self.tile_sumsq, self.tile_flag):
@@ -246,7 +238,6 @@ class ContiguousGradients:
             tf.zero_()
         if self.groups:
             self._boundary_stream = torch.cuda.current_stream(self.groups[0].device)
-        self.window += 1
 
     def remove(self) -> None:
         for h in self._handles:
