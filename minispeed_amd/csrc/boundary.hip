@@ -97,15 +97,15 @@ constexpr int kStatsBlocks = kStatsBlocksFixed;   // K2 partial slots per group
 // per mode.  Over the 1.3B fp16 gradients (292 segments), in isolation:
 // reading only, 8 waves x runs of 4 tiles x 4 units 0.398 ms (runs of
 // 1 / 2 / 8: 0.59 / 0.43 / 0.43; 4 waves: 0.43; 2 units: 0.41; fp32
-// gradients 0.822 ms, 2 units 0.841); writing, four waves per tile 1.25-1.27
+// gradients, runs of 4, 0.822 ms, 2 units 0.841); writing, four waves per tile 1.25-1.27
 // ms (one wave per tile x 2 units: 1.38; two slab sets and one barrier per
 // tile: 1.26-1.28).
 constexpr int kScanTile = MS_SCAN_TILE;
 #ifndef MS_SCAN_WAVES_READ
 #define MS_SCAN_WAVES_READ 8
 #endif
-#ifndef MS_SCAN_RUN_READ
-#define MS_SCAN_RUN_READ 4
+#ifndef MS_SCAN_RUN_KIB
+#define MS_SCAN_RUN_KIB 16
 #endif
 #ifndef MS_SCAN_DEPTH_READ
 #define MS_SCAN_DEPTH_READ 4
@@ -1632,14 +1632,20 @@ int scan_grid(int64_t ntiles, int tiles_per_block) {
   return static_cast<int>(g);
 }
 
-// Tiles per wave of the reading K1.  Runs of 2 and 4 tiles time alike over
-// 60K-640K tiles, runs of 1 up to 30% slower.  Up to kShortScanTiles tiles
-// every wave gets a tile of its own in one round of the chip; runs of 4 would
-// leave CUs idle and make each wave wait for four tiles in turn: K1 with its
-// fold over 0.8M params in 292 segments 18.6 -> 12.2 us, 3.3M in 52 15.6 ->
-// 11.2, 9.9M in 192 20.2 -> 16.5 (33M params, past the line: 22.7 us with
-// runs of 1 against 21.1).
-int scan_run_tiles(int64_t ntiles) { return ntiles <= kShortScanTiles ? 1 : MS_SCAN_RUN_READ; }
+// Tiles per wave of the reading K1: 16 KB of gradient, 4 tiles of 2-byte
+// elements or 2 of fp32.  fp16, runs of 1 / 2 / 4 tiles: 640,000 tiles 526 /
+// 453 / 422 us, 173,000 168 / 159 / 156, 60,762 85 / 88 / 89; fp32: 881 / 803 /
+// 871, 267 / 249 / 275, 127 / 124 / 137 (alone, every line of the cache dirty).
+// Up to kShortScanTiles tiles every wave gets a tile of its own in one round
+// of the chip; longer runs would leave CUs idle and make each wave wait for
+// several tiles in turn: K1 with its fold over 0.8M params in 292 segments
+// 18.6 -> 12.2 us, 3.3M in 52 15.6 -> 11.2, 9.9M in 192 20.2 -> 16.5 (33M
+// params, past the line: 22.7 us with runs of 1 against 21.1 with 4).
+template <class G>
+int scan_run_tiles(int64_t ntiles) {
+  constexpr int kRun = MS_SCAN_RUN_KIB * 1024 / (kScanTile * G::kBytes);
+  return ntiles <= kShortScanTiles ? 1 : kRun;
+}
 
 // the first of the tiles holding the last kCacheKeepBytes of gradient
 template <class G>
@@ -1652,7 +1658,7 @@ int64_t keep_from_tile(int64_t ntiles) {
 template <class G>
 void launch_buffer_stats(const ms_segment_t& one, double* tsum, uint32_t* tflag, hipStream_t st) {
   const int64_t n = one.numel, ntiles = scan_tiles(n);
-  const int run = scan_run_tiles(ntiles);
+  const int run = scan_run_tiles<G>(ntiles);
   hipLaunchKernelGGL((k_grad_stats<G, false, true, kScaleNone, true, true>),
                      dim3(scan_grid(ntiles, kScanWavesRead * run)), dim3(64 * kScanWavesRead), 0,
                      st, one, nullptr, 1, 0, n, 0, n, 1.0f, 1.0f, nullptr, tsum, tflag, ntiles, run,
@@ -1679,7 +1685,7 @@ void launch_stats_s(const ms_segment_t* segs, int nseg, int64_t begin, int64_t e
                          dim3(64 * kScanWavesFlat), 0, st, ms_segment_t{}, segs, nseg, begin, end,
                          ob, oe, mul, div, flat, tsum, tflag, ntiles, 1, keep_from);
     } else {
-      const int run = scan_run_tiles(ntiles);
+      const int run = scan_run_tiles<G>(ntiles);
       // the counted elements' flags from their sums wherever the scaling
       // cannot overflow a finite gradient (GradScan's kSumFlags)
       const bool sum_flags = kScale == kScaleNone ||
