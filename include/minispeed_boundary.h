@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MS_ABI_VERSION 9
+#define MS_ABI_VERSION 10
 
 /* groups one ms_boundary_scalars_noalloc call can scan, and the tiles
  * (MS_SCAN_TILE flat indices each) of the largest one: its static scratch
@@ -292,6 +292,44 @@ int ms_fused_adamw(float* master, float* exp_avg, float* exp_avg_sq,
                    int32_t nseg, int32_t grad_dtype, int32_t model_dtype,
                    int64_t begin, int64_t end, const ms_adamw_params_t* hp,
                    const ms_step_scalars_t* scalars, void* stream);
+
+/* One group's part of ms_boundary_step. */
+typedef struct ms_boundary_group {
+  const ms_segment_t* segs;      /* [dev] K1's table, tiles [0, numel); unused if scanned */
+  const ms_segment_t* own_segs;  /* [dev] K3's table, tiles [own_begin, own_end) */
+  int32_t nseg, own_nseg;
+  int32_t grad_dtype, model_dtype;
+  int64_t numel, own_begin, own_end;
+  float* flat_grad;              /* [dev, optional] K1 writes the fp32 flat gradient here */
+  float *master, *exp_avg, *exp_avg_sq;   /* [dev] fp32, index i at [i - own_begin] */
+  ms_adamw_params_t hp;          /* its grad_scale / unscale are K1's as well */
+  int32_t scanned;               /* non-zero: the tile slots are filled, no K1 */
+  int32_t reserved;              /* 0 */
+} ms_boundary_group_t;           /* 144 bytes */
+
+/* ms_norm_clip_tiles' arguments after the groups */
+typedef struct ms_norm_args {
+  double* block_sumsq;
+  uint32_t* block_flag;
+  int32_t nblk, has_clip, scaler_enabled, reserved;
+  double max_norm, scale;
+  int64_t good_steps, skipped_steps, window;
+  double min_scale, max_scale;
+  ms_step_scalars_t *out, *out_host;
+} ms_norm_args_t;                /* 104 bytes */
+
+/*
+ * The whole boundary in one call: ms_grad_tile_stats of every group that is
+ * not scanned, ms_norm_clip_tiles, then ms_fused_adamw (reading the raw
+ * gradients) of every group with a non-empty owned range; those functions'
+ * checks and results.
+ * groups, stats [host]: ngroups entries; stats[g] are group g's tile slots.
+ * events [host, optional]: hipEvent_t pairs recorded around each group's K1
+ *   (around nothing where it is scanned), K2 and each K3 that runs.
+ */
+int ms_boundary_step(const ms_boundary_group_t* groups, const ms_tile_stats_t* stats,
+                     int32_t ngroups, const ms_norm_args_t* norm, void* const* events,
+                     void* stream);
 
 /*
  * K4 — cast fp32 masters into model-dtype storage: flat [dev] holds index i

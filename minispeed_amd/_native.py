@@ -19,7 +19,7 @@ from typing import Optional
 import torch  # noqa: F401  (must precede the dlopen below, see module doc)
 
 LIB_NAME = "libminispeed_boundary.so"
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 DTYPE_F32 = 0
 DTYPE_F16 = 1
@@ -111,6 +111,51 @@ class TileStats(ctypes.Structure):
     ]
 
 
+class BoundaryGroup(ctypes.Structure):
+    """``ms_boundary_group_t``: one group of ms_boundary_step."""
+
+    _fields_ = [
+        ("segs", ctypes.c_void_p),
+        ("own_segs", ctypes.c_void_p),
+        ("nseg", ctypes.c_int32),
+        ("own_nseg", ctypes.c_int32),
+        ("grad_dtype", ctypes.c_int32),
+        ("model_dtype", ctypes.c_int32),
+        ("numel", ctypes.c_int64),
+        ("own_begin", ctypes.c_int64),
+        ("own_end", ctypes.c_int64),
+        ("flat_grad", ctypes.c_void_p),
+        ("master", ctypes.c_void_p),
+        ("exp_avg", ctypes.c_void_p),
+        ("exp_avg_sq", ctypes.c_void_p),
+        ("hp", AdamWParams),
+        ("scanned", ctypes.c_int32),
+        ("reserved", ctypes.c_int32),
+    ]
+
+
+class NormArgs(ctypes.Structure):
+    """``ms_norm_args_t``: K2's arguments in ms_boundary_step."""
+
+    _fields_ = [
+        ("block_sumsq", ctypes.c_void_p),
+        ("block_flag", ctypes.c_void_p),
+        ("nblk", ctypes.c_int32),
+        ("has_clip", ctypes.c_int32),
+        ("scaler_enabled", ctypes.c_int32),
+        ("reserved", ctypes.c_int32),
+        ("max_norm", ctypes.c_double),
+        ("scale", ctypes.c_double),
+        ("good_steps", ctypes.c_int64),
+        ("skipped_steps", ctypes.c_int64),
+        ("window", ctypes.c_int64),
+        ("min_scale", ctypes.c_double),
+        ("max_scale", ctypes.c_double),
+        ("out", ctypes.c_void_p),
+        ("out_host", ctypes.c_void_p),
+    ]
+
+
 class AccumRow(ctypes.Structure):
     """``ms_accum_row_t``: one gradient of ms_accumulate_grads."""
 
@@ -166,6 +211,11 @@ SIGNATURES = {
         ctypes.c_int,
         [_P, _P, _P, _P, _P, _I32, _I32, _I32, _I64, _I64,
          ctypes.POINTER(AdamWParams), _P, _P],
+    ),
+    "ms_boundary_step": (
+        ctypes.c_int,
+        [ctypes.POINTER(BoundaryGroup), ctypes.POINTER(TileStats), _I32, ctypes.POINTER(NormArgs),
+         _P, _P],
     ),
     "ms_cast_to_model": (ctypes.c_int, [_P, _I64, _I64, _P, _I32, _I32, _P]),
     "ms_accumulate_grad": (ctypes.c_int, [_P, _P, _I32, _I64, _I32, _P]),

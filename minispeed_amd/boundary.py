@@ -14,8 +14,8 @@ Replaces the unfused sequence of minispeed's
     (stage 3) free_parameters  stage_3.py:88-110   /
     DynamicLossScaler.update precision.py:50-62        K2 (checked on host)
 
-K3 is gated on the device overflow flag, so the launch sequence does not
-wait for the host: the only synchronisation is the final copy of the
+K3 is gated on the device overflow flag, so one call launches them all and
+does not wait for the host: the only synchronisation is the final copy of the
 ``ms_step_scalars_t`` K2 wrote.
 """
 
@@ -24,18 +24,13 @@ from __future__ import annotations
 import ctypes
 import time
 from dataclasses import dataclass
-from typing import Callable, List, Optional, Sequence, Tuple
+from typing import List, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
 
 from . import _native
 from .flat import FlatParamGroup, record_streams
-
-
-def _f32(x: float) -> float:
-    """x rounded to fp32 (round to nearest even), as a Python float."""
-    return ctypes.c_float(x).value
 
 
 def adamw_params(
@@ -129,24 +124,28 @@ class Workspace:
         self.tile_sums: Optional[torch.Tensor] = None
         self.tile_flags: Optional[torch.Tensor] = None
         self._tile_streams: set = set()
-        # every group's tile statistics, filled in for each call of K2
+        # the boundary call's arguments, filled in for each one
         self.tile_stats = (_native.TileStats * max(1, ngroups))()
+        self.groups = (_native.BoundaryGroup * max(1, ngroups))()
+        self.norm = _native.NormArgs(
+            block_sumsq=self.partials.data_ptr(), block_flag=self.flags.data_ptr(),
+            nblk=self.nblk, out=self.scalars.data_ptr())
         # K2 also writes its result to pinned host memory, which the host
         # polls (HostReadback): no copy, and K3, queued behind K2, keeps
         # running while the host does its bookkeeping
         self.readback = HostReadback()
+        self.norm.out_host = self.readback.ptr
         self._stream: Optional[torch.cuda.Stream] = None   # stream of the last boundary
 
-    def tile_ptrs(self, ntiles: int):
+    def tile_ptrs(self, ntiles: int, cur: torch.cuda.Stream):
         """Addresses (sums, flags) of at least ``ntiles`` K1 tile slots for
-        kernels on the current stream."""
+        kernels on the current stream ``cur``."""
         if self.tile_sums is None or self.tile_sums.numel() < ntiles:
             # the replaced buffers' memory stays with the streams recorded on
             # them until those have run what was queued there
             self.tile_sums = torch.empty(max(1, ntiles), dtype=torch.float64, device=self.device)
             self.tile_flags = torch.empty(max(1, ntiles), dtype=torch.int32, device=self.device)
             self._tile_streams = set()
-        cur = torch.cuda.current_stream(self.device)
         if cur.cuda_stream not in self._tile_streams:
             self.tile_sums.record_stream(cur)
             self.tile_flags.record_stream(cur)
@@ -216,6 +215,16 @@ class LaunchTimer:
         name, start = token
         self._events.setdefault(name, []).append((start, self._record()))
 
+    def pairs(self, names: Sequence[str]):
+        """An event pair for every name, in order, as the array that
+        ms_boundary_step records."""
+        events = (ctypes.c_void_p * (2 * len(names)))()
+        for k, name in enumerate(names):
+            a, b = (self._pool.pop() if self._pool else self._create() for _ in range(2))
+            events[2 * k], events[2 * k + 1] = a, b
+            self._events.setdefault(name, []).append((a, b))
+        return events
+
     def durations_ms(self, name: str) -> List[float]:
         out = []
         for a, b in self._events.get(name, []):
@@ -238,17 +247,6 @@ class LaunchTimer:
             hip.hipEventDestroy(ev)
 
 
-class _NoTimer:
-    def start(self, name):
-        return None
-
-    def stop(self, token):
-        return None
-
-
-_NO_TIMER = _NoTimer()
-
-
 @dataclass
 class GroupLaunch:
     """What K1/K3 need for one group at one boundary."""
@@ -261,48 +259,66 @@ class GroupLaunch:
     step: int                     # Adam step number this update would use
     exp_avg: torch.Tensor         # owned-range moments (optim/adam.py:58-65)
     exp_avg_sq: torch.Tensor
-    grads: Sequence[int]          # gradient address per parameter (0: none)
+    rows: Optional[object]        # the group's BoundaryRows with its gradients, or
+    grads: Optional[Sequence[int]]   # (a shard) the address per parameter (0: none)
     grad_dtype: Optional[int] = None   # MS_DTYPE_* of the gradients (default: the params')
     # (sum-of-squares slots, flag slots, count) K5 left for the gradients
     # (contiguous mode): folded into the partial sums instead of the K1 scan
     tile_stats: Optional[Tuple[int, int, int]] = None
 
 
+def _tables(gl: GroupLaunch, write_model: bool, gbytes: int, cur: torch.cuda.Stream):
+    """K1's and K3's (table address, rows): one table where the group has
+    :meth:`FlatParamGroup.boundary_rows`, one each for a shard."""
+    g = gl.group
+    if gl.rows is not None:
+        # ZeRO-3 placeholders are sized as the parameters unless someone
+        # replaced one; the general table looks at what each one covers
+        if gl.rows.models(write_model, g._partitioned) < 0:
+            t = g.table("k1").upload(gl.rows.table, cur)
+            return t, t
+        g.model_pointers()     # raises, unless it is the size
+        if gl.grads is None:
+            gl.grads = np.zeros(len(g.params) + 1, dtype=np.int64)
+            gl.grads[g._whole_rows()[1]] = gl.rows.table[:, 2]
+    mptrs = g.model_pointers() if write_model else None
+    lo, hi = g.own_range
+    t1 = g.table("k1").upload(g.boundary_table(0, g.numel_padded, gl.grads, None, gbytes), cur)
+    if hi <= lo:
+        return t1, (None, 0)
+    return t1, g.table("k3").upload(g.boundary_table(lo, hi, gl.grads, mptrs, gbytes), cur)
+
+
 def run_boundary(
     launches: List[GroupLaunch],
     ws: Workspace,
+    cur: torch.cuda.Stream,
     *,
     scaler,
     max_norm: Optional[float],
     materialize_flat_grad: bool,
-    model_targets: Callable[[], List[Optional[List[int]]]],
+    write_model: bool,
     timer: Optional[LaunchTimer] = None,
     keep: Sequence[Optional[torch.Tensor]] = (),
 ) -> _native.StepScalars:
-    """Launch the whole boundary and return K2's scalars (one host sync).
+    """Launch the whole boundary on ``cur`` (the stream ``ws.enter()``
+    returned) and return K2's scalars (one host sync).
 
-    K1 per group and K2 with the folds it needs are launched as soon as the
-    gradient addresses are known (K2 writes its scalars to device memory for
-    K3 and to pinned host memory for the host); ``model_targets()``
-    (the addresses K3 casts the updated masters into, per group; ``None`` for
-    no write) is called after that, so whatever it does on the host overlaps
-    K1 on the device.  The function returns once K2's scalars are on the
-    host, which is before K3 has finished: K3 runs on the current stream, so
-    everything queued there afterwards is ordered after it.  ``keep`` holds
-    the tensors behind ``GroupLaunch.grads``; the current stream is recorded
-    on each, so the caller may drop them once this returns, whichever
-    stream allocated them.
+    One table per group serves K1 and K3 and one call launches every kernel
+    (ms_boundary_step): a table and a call per kernel took the host 25 us more
+    at every boundary, all of a small model's step.  ``write_model``: K3 casts
+    the updated masters into the parameters' storage.  The function returns
+    once K2's scalars are on the host, which is before K3 has finished: K3
+    runs on ``cur``, so everything queued there afterwards is ordered after
+    it.  ``keep`` holds the tensors behind ``GroupLaunch.grads``; ``cur`` is
+    recorded on each, so the caller may drop them once this returns,
+    whichever stream allocated them (``GroupLaunch.rows`` has recorded it on
+    its own).
     """
     lib = _native.load()
-    device = ws.device
-    cur = ws.enter()
-    stream = cur.cuda_stream
     scale = float(scaler.loss_scale_factor)
     unscale = scale != 1.0
-    scale32 = _f32(scale)
-    timer = timer or _NO_TIMER
 
-    dtypes = []
     # a group whose accumulation pass already scanned the sums has its tile
     # statistics (no second read of the sums); the others' tile slots lie one
     # region after another, K2 reads them all
@@ -310,83 +326,58 @@ def run_boundary(
                and gl.group.own_range == (0, gl.group.numel_padded) for gl in launches]
     ntiles = [0 if done else _native.scan_tiles(gl.group.numel_padded)
               for gl, done in zip(launches, scanned)]
-    tsum, tflag = ws.tile_ptrs(sum(ntiles))
-    stats = ws.tile_stats
-    for gi, gl in enumerate(launches):
-        g = gl.group
-        dtype = _native.ms_dtype(g.params[0].dtype)
-        gdtype = dtype if gl.grad_dtype is None else gl.grad_dtype
-        flat_out = None
-        if materialize_flat_grad:
-            flat_out = g.flat_grad_for_overwrite()      # K1 writes every element
-        lo, hi = g.own_range
-        gbytes = 4 if gdtype == _native.DTYPE_F32 else 2
-        if scanned[gi]:
-            tok = timer.start("k1")          # nothing to launch
-            stats[gi].sumsq, stats[gi].flag, stats[gi].ntiles = gl.tile_stats
-            timer.stop(tok)
-        else:
-            t1 = g.table("k1").upload(g.boundary_table(0, g.numel_padded, gl.grads, None, gbytes), cur)
-            tok = timer.start("k1")
-            rc = lib.ms_grad_tile_stats(
-                t1[0], t1[1], gdtype, 0, g.numel_padded, lo, hi,
-                _native.SCALE_DIVIDE if unscale else _native.SCALE_NONE, scale32,
-                flat_out.data_ptr() if flat_out is not None else None,
-                tsum, tflag, ntiles[gi], stream,
-            )
-            timer.stop(tok)
-            _native.check(rc, "ms_grad_tile_stats")
-            stats[gi].sumsq, stats[gi].flag, stats[gi].ntiles = tsum, tflag, ntiles[gi]
-            tsum += 8 * ntiles[gi]
-            tflag += 4 * ntiles[gi]
-        dtypes.append((gdtype, dtype, gbytes))
-
-    ws.readback.arm()
-    tok = timer.start("k2")
-    rc = lib.ms_norm_clip_tiles(
-        stats, len(launches), ws.partials.data_ptr(), ws.flags.data_ptr(), ws.nblk,
-        1 if max_norm is not None else 0, float(max_norm or 0.0),
-        1 if scaler.enabled else 0, float(scaler.scale), int(scaler.good_steps),
-        int(scaler.skipped_steps), int(scaler.scale_window),
-        float(scaler.min_scale), float(scaler.max_scale),
-        ws.scalars.data_ptr(), ws.readback.ptr, stream,
-    )
-    timer.stop(tok)
-    _native.check(rc, "ms_norm_clip_tiles")
-
-    models = model_targets()
-    for gl, (gdtype, dtype, gbytes), mptrs in zip(launches, dtypes, models):
+    tsum, tflag = ws.tile_ptrs(sum(ntiles), cur)
+    for b, st, gl, done, nt in zip(ws.groups, ws.tile_stats, launches, scanned, ntiles):
         g = gl.group
         lo, hi = g.own_range
-        if hi <= lo:
-            continue
         master = g.shard
-        if master.numel() != hi - lo or gl.exp_avg.numel() != hi - lo or gl.exp_avg_sq.numel() != hi - lo:
+        if hi > lo and not (master.numel() == gl.exp_avg.numel() == gl.exp_avg_sq.numel() == hi - lo):
             raise RuntimeError(
                 f"grad/shard shape mismatch: owned range {hi - lo} vs master {master.numel()}, "
                 f"moments {gl.exp_avg.numel()}/{gl.exp_avg_sq.numel()}"
             )
-        t3 = g.table("k3").upload(g.boundary_table(lo, hi, gl.grads, mptrs, gbytes), cur)
-        # K3 reads the gradients themselves also where K1 wrote the fp32 flat
-        # gradient: its unscale rounds exactly as K1's, and 2-byte gradients
-        # are 2 B/param less to read than the flat copy (350M fp16 params:
-        # K3 1.77 -> 1.54 ms)
-        hp = adamw_params(gl.lr, gl.betas, gl.eps, gl.weight_decay, gl.step,
-                          grad_scale=scale, unscale=unscale)
-        tok = timer.start("k3")
-        rc = lib.ms_fused_adamw(
-            master.data_ptr(), gl.exp_avg.data_ptr(), gl.exp_avg_sq.data_ptr(), None,
-            t3[0], t3[1], gdtype, dtype, lo, hi, ctypes.byref(hp), ws.scalars.data_ptr(), stream,
-        )
-        timer.stop(tok)
-        _native.check(rc, "ms_fused_adamw")
+        b.model_dtype = _native.ms_dtype(g.params[0].dtype)
+        b.grad_dtype = gdtype = b.model_dtype if gl.grad_dtype is None else gl.grad_dtype
+        (b.segs, b.nseg), (b.own_segs, b.own_nseg) = _tables(
+            gl, write_model, 4 if gdtype == _native.DTYPE_F32 else 2, cur)
+        b.numel, b.own_begin, b.own_end = g.numel_padded, lo, hi
+        # K1 writes every element; K3 reads the gradients themselves also
+        # then: its unscale rounds exactly as K1's, and 2-byte gradients are
+        # 2 B/param less to read than the flat copy (350M fp16 params: K3
+        # 1.77 -> 1.54 ms)
+        b.flat_grad = g.flat_grad_for_overwrite().data_ptr() if materialize_flat_grad else None
+        b.master, b.exp_avg, b.exp_avg_sq = (
+            master.data_ptr(), gl.exp_avg.data_ptr(), gl.exp_avg_sq.data_ptr())
+        b.hp = adamw_params(gl.lr, gl.betas, gl.eps, gl.weight_decay, gl.step,
+                            grad_scale=scale, unscale=unscale)
+        b.scanned = done
+        if done:
+            st.sumsq, st.flag, st.ntiles = gl.tile_stats
+        else:
+            st.sumsq, st.flag, st.ntiles = tsum, tflag, nt
+            tsum += 8 * nt
+            tflag += 4 * nt
 
-    # The gradients may come from another stream (the one backward ran on):
-    # once the caller drops them, the caching allocator could hand their
-    # memory to that stream while K1 / K3 still read it here.  Recording
-    # this stream on them defers the reuse until everything queued here so
-    # far has run.  Done while K1 / K2 run, before the host waits.
-    record_streams(keep, cur)
+    norm = ws.norm
+    norm.has_clip, norm.max_norm = (0, 0.0) if max_norm is None else (1, float(max_norm))
+    norm.scaler_enabled, norm.scale = bool(scaler.enabled), float(scaler.scale)
+    norm.good_steps, norm.skipped_steps = int(scaler.good_steps), int(scaler.skipped_steps)
+    norm.window = int(scaler.scale_window)
+    norm.min_scale, norm.max_scale = float(scaler.min_scale), float(scaler.max_scale)
+    events = None
+    if timer is not None:
+        k3 = sum(gl.group.own_range[1] > gl.group.own_range[0] for gl in launches)
+        events = timer.pairs(["k1"] * len(launches) + ["k2"] + ["k3"] * k3)
+    # Gradients may come from another stream (the one backward ran on): once
+    # the caller drops them, the caching allocator could hand their memory to
+    # that stream while K1 / K3 still read it here.  Recording this stream on
+    # them defers the reuse until everything queued here by then has run.
+    if keep:
+        record_streams(keep, cur)
+    ws.readback.arm()
+    rc = lib.ms_boundary_step(ws.groups, ws.tile_stats, len(launches), ctypes.byref(norm), events,
+                              cur.cuda_stream)
+    _native.check(rc, "ms_boundary_step")
     return ws.finish_readback()
 
 

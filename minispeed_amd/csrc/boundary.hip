@@ -2100,6 +2100,46 @@ int ms_fused_adamw(float* master, float* exp_avg, float* exp_avg_sq,
   return launch_status();
 }
 
+int ms_boundary_step(const ms_boundary_group_t* groups, const ms_tile_stats_t* stats,
+                     int32_t ngroups, const ms_norm_args_t* norm, void* const* events,
+                     void* stream) {
+  if (ngroups < 0 || (ngroups > 0 && (!groups || !stats)) || !norm) return MS_EINVAL;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  auto mark = [&]() -> int {
+    if (!events) return MS_OK;
+    return static_cast<int>(hipEventRecord(static_cast<hipEvent_t>(*events++), st));
+  };
+  int rc = MS_OK;
+  for (int32_t g = 0; g < ngroups; ++g) {
+    const ms_boundary_group_t& b = groups[g];
+    if ((rc = mark()) != MS_OK) return rc;
+    if (!b.scanned) {
+      rc = ms_grad_tile_stats(b.segs, b.nseg, b.grad_dtype, 0, b.numel, b.own_begin, b.own_end,
+                              b.hp.unscale, b.hp.grad_scale, b.flat_grad,
+                              const_cast<double*>(stats[g].sumsq),
+                              const_cast<uint32_t*>(stats[g].flag), stats[g].ntiles, stream);
+      if (rc != MS_OK) return rc;
+    }
+    if ((rc = mark()) != MS_OK) return rc;
+  }
+  if ((rc = mark()) != MS_OK) return rc;
+  rc = ms_norm_clip_tiles(stats, ngroups, norm->block_sumsq, norm->block_flag, norm->nblk,
+                          norm->has_clip, norm->max_norm, norm->scaler_enabled, norm->scale,
+                          norm->good_steps, norm->skipped_steps, norm->window, norm->min_scale,
+                          norm->max_scale, norm->out, norm->out_host, stream);
+  if (rc != MS_OK || (rc = mark()) != MS_OK) return rc;
+  for (int32_t g = 0; g < ngroups; ++g) {
+    const ms_boundary_group_t& b = groups[g];
+    if (b.own_end <= b.own_begin) continue;
+    if ((rc = mark()) != MS_OK) return rc;
+    rc = ms_fused_adamw(b.master, b.exp_avg, b.exp_avg_sq, nullptr, b.own_segs, b.own_nseg,
+                        b.grad_dtype, b.model_dtype, b.own_begin, b.own_end, &b.hp, norm->out,
+                        stream);
+    if (rc != MS_OK || (rc = mark()) != MS_OK) return rc;
+  }
+  return MS_OK;
+}
+
 int ms_accumulate_grads(const ms_accum_row_t* rows, int32_t nrows, int32_t src_dtype,
                         int32_t unscale, float grad_scale, void* stream) {
   if (!valid_dtype(src_dtype) || nrows < 0 || (nrows > 0 && !rows)) return MS_EINVAL;

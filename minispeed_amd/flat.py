@@ -229,10 +229,12 @@ class SegmentTable:
             return 0, 0
         if stream is None:
             stream = torch.cuda.current_stream(self.device)
-        for k, entry in enumerate(self._entries):
-            host, dev, seen = entry
-            if host.shape == table.shape and np.array_equal(host, table):
-                self._entries.append(self._entries.pop(k))
+        same = _walk().same_table
+        for k in range(len(self._entries) - 1, -1, -1):
+            host, dev, seen = self._entries[k]
+            if same(host, table):
+                if k != len(self._entries) - 1:
+                    self._entries.append(self._entries.pop(k))
                 if stream.cuda_stream not in seen:
                     dev.record_stream(stream)
                     seen.add(stream.cuda_stream)
@@ -611,6 +613,7 @@ class FlatParamGroup:
         self._shard_dirty = False
         self._tables = {}
         self._rows = None   # static (begin, numel) rows of the whole-range table
+        self._native_rows = None   # the boundary's table over them
         self._device_index = device.index if device.index is not None else torch.cuda.current_device()
 
     # ------------------------------------------------------------- ranges
@@ -908,20 +911,7 @@ class FlatParamGroup:
         if mptrs is not None and self._partitioned:   # ZeRO-3 placeholders may be slices
             full = all(p.numel() == n for p, n in zip(self.params, self._numels))
         if lo == 0 and hi == self.numel_padded and full:
-            if self._rows is None:
-                rows, idx = [], []
-                for i, (off, n) in enumerate(zip(self.layout.offsets, self._numels)):
-                    if n:
-                        rows.append((off, n))
-                        idx.append(i)
-                if self.numel_padded > self.numel:
-                    rows.append((self.numel, self.numel_padded - self.numel))
-                    idx.append(n_params)
-                base = np.zeros((len(rows), 4), dtype=np.int64)
-                base[:, :2] = np.asarray(rows, dtype=np.int64).reshape(-1, 2)
-                check_table(base, 0, self.numel_padded)
-                self._rows = (base, np.asarray(idx, dtype=np.int64))
-            base, idx = self._rows
+            base, idx = self._whole_rows()
             table = base.copy()
             if gptrs is not None:
                 table[:, 2] = _with_pad_slot(gptrs, n_params)[idx]
@@ -939,6 +929,41 @@ class FlatParamGroup:
         table = self.layout.segments(lo, hi, grads, models)
         check_table(table, lo, hi)
         return table
+
+    def _whole_rows(self) -> Tuple[np.ndarray, np.ndarray]:
+        """The whole padded range's rows without addresses, and the parameter
+        of each (their count: the padding row)."""
+        if self._rows is None:
+            rows, idx = [], []
+            for i, (off, n) in enumerate(zip(self.layout.offsets, self._numels)):
+                if n:
+                    rows.append((off, n))
+                    idx.append(i)
+            if self.numel_padded > self.numel:
+                rows.append((self.numel, self.numel_padded - self.numel))
+                idx.append(len(self.params))
+            base = np.zeros((len(rows), 4), dtype=np.int64)
+            base[:, :2] = np.asarray(rows, dtype=np.int64).reshape(-1, 2)
+            check_table(base, 0, self.numel_padded)
+            self._rows = (base, np.asarray(idx, dtype=np.int64))
+        return self._rows
+
+    def boundary_rows(self):
+        """The table K1 and K3 share where the owned range is the whole
+        padded range (a ``_walk.BoundaryRows``, refilled at each boundary);
+        ``None`` for a shard, whose K3 has a table of its own."""
+        if not self.whole_range:
+            return None
+        if self._native_rows is None:
+            base, idx = self._whole_rows()
+            self._native_rows = _walk().BoundaryRows(self.params, self._numels, self._device_index,
+                                                     base.copy(), idx.tolist())
+        return self._native_rows
+
+    def drop_rows(self) -> None:
+        """Let go of the gradients that :meth:`boundary_rows` holds."""
+        if self._native_rows is not None:
+            self._native_rows.drop()
 
     # ----------------------------------------------------------- grads
     @property
@@ -969,8 +994,7 @@ class FlatParamGroup:
         return self._grad
 
     def release_grads(self) -> None:
-        for p in self.params:
-            p.grad = None
+        _walk().release_grads(self.params)
 
     @torch.no_grad()
     def flatten_grads(self) -> None:

@@ -32,7 +32,9 @@ class ZeROOptimizer:
         self.rank = comm.get_rank()
         self.adam = FlatAdam(flat_groups, option_groups, zero_stage=zero_stage)
         self.grad_norm: Optional[float] = None
-        self._workspace: Optional[Workspace] = None
+        self._workspace = Workspace(flat_groups[0].device, len(flat_groups)) if flat_groups else None
+        for g in flat_groups:
+            g.boundary_rows()      # laid out before the first boundary
         self.launch_timer: Optional[LaunchTimer] = None  # HIP-event timing hook
         # opt-in fp32 gradient accumulation (contiguous.py); set by the engine
         self.contiguous = None
@@ -103,15 +105,10 @@ class ZeROOptimizer:
         return self.adam.step()
 
     # ------------------------------------------------------ fused boundary
-    def _ws(self) -> Workspace:
-        if self._workspace is None:
-            self._workspace = Workspace(self.flat_groups[0].device, len(self.flat_groups))
-        return self._workspace
-
-    def _model_targets(self) -> List[Optional[List[int]]]:
-        """Where K3 writes the model-dtype copy of each group (addresses of
-        the parameters' storage)."""
-        return [g.model_pointers() for g in self.flat_groups]
+    def _model_targets(self) -> bool:
+        """Ready the parameters for K3's cast into their storage; whether it
+        writes them."""
+        return True
 
     def _after_boundary(self, overflow: bool) -> None:
         """Stage-specific follow-up once the scalars are on the host."""
@@ -125,39 +122,45 @@ class ZeROOptimizer:
         Adam step counters advance only for an applied step (the caller
         commits them via :meth:`commit_step`).
         """
-        ws = self._ws()
-        keep: List[torch.Tensor] = []
-        launches = []
-        for gi, (g, group, state) in enumerate(zip(self.flat_groups, self.adam.param_groups,
-                                                   self.adam.state)):
-            grad_dtype = None
-            tile_stats = None
-            if self.contiguous is not None:
-                ptrs, grad_dtype = self.contiguous.grad_pointers(gi), _native.DTYPE_F32
-                tile_stats = self.contiguous.tile_stats(gi, scaler.loss_scale_factor)
-            else:
-                ptrs, tensors, grad_dtype = g.grad_pointers()
-                keep.extend(tensors)
-            lr, betas, eps, wd = FlatAdam.hyper(group)
-            launches.append(GroupLaunch(
-                group=g, lr=lr, betas=betas, eps=eps, weight_decay=wd,
-                step=state["step"] + 1, exp_avg=state["exp_avg"], exp_avg_sq=state["exp_avg_sq"],
-                grads=ptrs, grad_dtype=grad_dtype, tile_stats=tile_stats,
-            ))
-
-        def model_targets():
-            # runs while K1 is on the device: release param.grad (flat.py:213)
-            # and collect the cast targets
+        ws = self._workspace
+        cur = ws.enter()
+        stream = int(cur.device_type), int(cur.device_index), int(cur.stream_id)
+        try:
+            keep: List[torch.Tensor] = []
+            launches = []
+            for gi, (g, group, state) in enumerate(zip(self.flat_groups, self.adam.param_groups,
+                                                       self.adam.state)):
+                grad_dtype = None
+                tile_stats = None
+                ptrs = None
+                rows = g.boundary_rows()
+                if self.contiguous is not None:
+                    ptrs, grad_dtype = self.contiguous.grad_pointers(gi), _native.DTYPE_F32
+                    tile_stats = self.contiguous.tile_stats(gi, scaler.loss_scale_factor)
+                elif rows is None or rows.grads(*stream) >= 0:
+                    ptrs, tensors, grad_dtype = g.grad_pointers()
+                    keep.extend(tensors)
+                if rows is not None and ptrs is not None:
+                    rows.set_grads(ptrs)
+                lr, betas, eps, wd = FlatAdam.hyper(group)
+                launches.append(GroupLaunch(
+                    group=g, lr=lr, betas=betas, eps=eps, weight_decay=wd,
+                    step=state["step"] + 1, exp_avg=state["exp_avg"], exp_avg_sq=state["exp_avg_sq"],
+                    rows=rows, grads=ptrs, grad_dtype=grad_dtype, tile_stats=tile_stats,
+                ))
+            # release param.grad (flat.py:213); `rows` and `keep` hold what the
+            # kernels read
             for g in self.flat_groups:
                 g.release_grads()
-            return self._model_targets()
-
-        scalars = run_boundary(
-            launches, ws, scaler=scaler, max_norm=max_norm,
-            materialize_flat_grad=materialize_flat_grad, model_targets=model_targets,
-            timer=self.launch_timer, keep=keep,
-        )
-        del keep  # recorded on the boundary's stream by run_boundary
+            scalars = run_boundary(
+                launches, ws, cur, scaler=scaler, max_norm=max_norm,
+                materialize_flat_grad=materialize_flat_grad, write_model=self._model_targets(),
+                timer=self.launch_timer, keep=keep,
+            )
+        finally:
+            # (the boundary's stream is recorded on every gradient)
+            for g in self.flat_groups:
+                g.drop_rows()
         overflow = bool(scalars.overflow)
         if not overflow:
             self.grad_norm = float(scalars.norm)

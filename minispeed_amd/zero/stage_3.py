@@ -25,7 +25,7 @@ instead.
 
 from __future__ import annotations
 
-from typing import List, Optional
+from typing import List
 
 import torch
 
@@ -89,15 +89,14 @@ class ZeROStage3Optimizer(ZeROOptimizer):
         for g in self.flat_groups:
             g.grad = None
 
-    def _model_targets(self) -> List[Optional[List[int]]]:
-        if not self._gathered:
-            # the reference's free_parameters is a no-op then: nothing written
-            self._boundary_freed = False
-            return [None for _ in self.flat_groups]
-        for g in self.flat_groups:
-            g.dematerialize_params()
-        self._boundary_freed = True
-        return [g.model_pointers() for g in self.flat_groups]
+    def _model_targets(self) -> bool:
+        # not gathered: the reference's free_parameters is a no-op then,
+        # nothing is written
+        self._boundary_freed = self._gathered
+        if self._gathered:
+            for g in self.flat_groups:
+                g.dematerialize_params()
+        return self._boundary_freed
 
     def _after_boundary(self, overflow: bool) -> None:
         if self._boundary_freed:
