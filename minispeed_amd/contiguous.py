@@ -17,8 +17,8 @@ The same K5 pass also does the boundary scan's work on the new sums: for
 every 2048-element tile of a parameter's slice it writes the fp64 sum of
 squares of the unscaled sums and an inf/nan flag into the tile's slot.
 The last K5 that touched a tile always left the statistics of its current
-sums, and the slots are zeroed when a window starts (parameters without a
-gradient count as zeros), so at the boundary the slots are folded into the
+sums, and the slots of parameters without a gradient in the window are zeros
+at its boundary, so there the slots are folded into the
 norm's partial sums (``ms_reduce_tile_stats``) and the fp32 sums are not
 read a second time: the boundary moves 30 B/param (K3) instead of 34.
 When the loss scale that unscaled the statistics is not the boundary's
@@ -124,8 +124,8 @@ class ContiguousGradients:
         # the (unscale, fp32 scale) of this window's flushes; None before the
         # first, False once two differed
         self._window_unscale = None
-        # the stream of the last boundary (the sums and slots were read and
-        # cleared there): a flush on another stream waits for it first
+        # the stream of the last boundary (the sums and slots were read
+        # there): a flush on another stream waits for it first
         self._boundary_stream: Optional[torch.cuda.Stream] = None
         self._callback_pending = False
         self._handles = []
@@ -223,19 +223,21 @@ class ContiguousGradients:
         w = self._window_unscale
         if w is False or (w is not None and w != unscale_of(float(scale))):
             return None
+        # every K5 of this window wrote all slots of its parameter; what an
+        # earlier window left for the others is cleared here, once (clearing
+        # every slot at every window took two launches a group)
+        for begin, end in self._queue.stale_slots(gi, _native.ACCUM_TILE):
+            self.tile_sumsq[gi][begin:end].zero_()
+            self.tile_flag[gi][begin:end].zero_()
         return (self.tile_sumsq[gi].data_ptr(), self.tile_flag[gi].data_ptr(),
                 int(self.tile_sumsq[gi].numel()))
 
     def next_window(self) -> None:
-        """Forget the sums (the boundary consumed them, or zero_grad): the
-        statistics slots are cleared on the current stream; queued
+        """Forget the sums (the boundary consumed them, or zero_grad); queued
         gradients of the abandoned window are dropped unread."""
         self._queue.next_window()
         self._callback_pending = False
         self._window_unscale = None
-        for ts, tf in zip(self.tile_sumsq, self.tile_flag):
-            ts.zero_()
-            tf.zero_()
         if self.groups:
             self._boundary_stream = torch.cuda.current_stream(self.groups[0].device)
 

@@ -15,6 +15,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 #include <pybind11/numpy.h>
+#include <pybind11/stl.h>
 
 #include <c10/core/Stream.h>
 #include <c10/core/impl/VirtualGuardImpl.h>
@@ -285,7 +286,7 @@ class GradQueue {
     }
     Group g{device_index, accum, sumsq, flag, {}};
     for (size_t k = 0; k < numels.size(); ++k) {
-      g.params.push_back({numels[k], offsets[k], tile0[k], -1, false});
+      g.params.push_back({numels[k], offsets[k], tile0[k], -1, false, false});
     }
     groups_.push_back(std::move(g));
   }
@@ -326,7 +327,7 @@ class GradQueue {
   bool empty() const { return entries_.empty(); }
 
   // The queue's content as [(device index, MS_DTYPE_*, rows, gradients)], one
-  // item per device and dtype in the order of their first entries; rows are
+  // item per device and dtype, in the order of their first entries; rows are
   // ms_accum_row_t records (48 bytes).  The queue is empty afterwards.
   py::list rows() {
     struct Batch {
@@ -376,6 +377,24 @@ class GradQueue {
     }
   }
 
+  // The slot ranges [begin, end) that still hold an earlier window's
+  // statistics, of parameters without a gradient in this one; they count as
+  // cleared from here on.
+  std::vector<std::pair<int64_t, int64_t>> stale_slots(int64_t gi, int64_t tile) {
+    std::vector<std::pair<int64_t, int64_t>> out;
+    for (Param& p : groups_.at(gi).params) {
+      if (!p.stats || p.seen == window_) continue;
+      p.stats = false;
+      const int64_t end = p.tile0 + (p.numel + tile - 1) / tile;
+      if (!out.empty() && out.back().second == p.tile0) {
+        out.back().second = end;
+      } else if (end > p.tile0) {
+        out.emplace_back(p.tile0, end);
+      }
+    }
+    return out;
+  }
+
   // Drop what is queued and start the next window.
   void next_window() {
     for (const Entry& e : entries_) groups_[e.group].params[e.index].queued = false;
@@ -390,6 +409,7 @@ class GradQueue {
   struct Param {
     int64_t numel, offset, tile0, seen;   // seen: the window it last contributed in
     bool queued;
+    bool stats;   // its slots hold statistics (not zeros)
   };
   struct Group {
     int64_t device, accum, sumsq, flag;
@@ -413,7 +433,7 @@ class GradQueue {
     Param& p = groups_[gi].params[k];
     entries_.push_back({gi, k, g, p.seen != window_});
     p.seen = window_;
-    p.queued = true;
+    p.queued = p.stats = true;
     queued_ += p.numel;
   }
 
@@ -450,5 +470,6 @@ PYBIND11_MODULE(_walk, m) {
       .def("empty", &GradQueue::empty)
       .def("rows", &GradQueue::rows)
       .def("pointers", &GradQueue::pointers)
+      .def("stale_slots", &GradQueue::stale_slots)
       .def("next_window", &GradQueue::next_window);
 }

@@ -82,3 +82,24 @@ def test_left_to_the_caller():
     with pytest.raises(IndexError):
         q.take(1, 0, p)
     assert q.empty()
+
+
+def test_slots_that_an_earlier_window_left():
+    q = _queue()
+    assert q.stale_slots(0, 2048) == []
+    for k in range(3):
+        q.put(0, k, torch.zeros(SIZES[k]))
+    q.rows()
+    assert q.stale_slots(0, 2048) == []               # all of this window
+    q.next_window()
+    q.put(0, 2, torch.zeros(4100))
+    q.rows()
+    assert q.stale_slots(0, 2048) == [(0, 1)]
+    q.next_window()
+    assert q.stale_slots(0, 2048) == [(1, 4)]         # the first one stays clear
+    assert q.stale_slots(0, 2048) == []
+    q.put(0, 0, torch.zeros(5))
+    q.put(0, 2, torch.zeros(4100))
+    q.rows()
+    q.next_window()
+    assert q.stale_slots(0, 2048) == [(0, 4)]         # neighbours in one range
