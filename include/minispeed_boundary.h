@@ -372,14 +372,16 @@ typedef struct ms_accum_row {
 } ms_accum_row_t;       /* 48 bytes */
 
 /* Rows per K5 launch of ms_accumulate_grads (they travel in the kernel
- * arguments, so a batch needs no device-side table), and the elements one
- * K5 tile (one statistics slot) covers. */
-#define MS_ACCUM_ROWS_PER_LAUNCH 64
+ * arguments, so a batch needs no device-side table), where their slices and
+ * slots lie within 8 GiB of one of four (64 where they do not), and the
+ * elements one K5 tile (one statistics slot) covers. */
+#define MS_ACCUM_ROWS_PER_LAUNCH 152
 #define MS_ACCUM_TILE 2048
 
 /*
  * K5, batched: ms_accumulate_grad for every row of rows[0 .. nrows) [host
- * memory, read before the call returns], ceil(nrows / 64) launches.  Rows
+ * memory, read before the call returns], one launch per
+ * MS_ACCUM_ROWS_PER_LAUNCH rows.  Rows
  * with numel 0 are skipped; the dst ranges of one call must not overlap.
  * The contiguous-gradient hooks queue the gradients backward produces and
  * flush them through this call (at the end of backward, or when a bucket

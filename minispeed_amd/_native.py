@@ -170,7 +170,7 @@ class AccumRow(ctypes.Structure):
     ]
 
 
-ACCUM_ROWS_PER_LAUNCH = 64
+ACCUM_ROWS_PER_LAUNCH = 152
 ACCUM_TILE = 2048
 # flat indices per K1 tile (MS_SCAN_TILE)
 SCAN_TILE = 2048

@@ -7,7 +7,7 @@ With ``"hip_boundary": {"contiguous_gradients": true}`` a post-accumulate-grad
 hook on every parameter takes the gradient backward has just produced and
 releases ``param.grad``; the queued gradients are added, in fp32, into the
 parameters' slices of one flat buffer per group by K5 in batches
-(``ms_accumulate_grads``, up to 64 gradients per launch): when a bucket of
+(``ms_accumulate_grads``, up to 152 gradients per launch): when a bucket of
 queued elements fills, and at the end of every backward pass (an autograd
 final callback).  K5 runs on the stream current when the batch is flushed:
 the gradients of one backward are assumed to come from that stream, as

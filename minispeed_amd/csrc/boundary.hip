@@ -1392,7 +1392,7 @@ __global__ __launch_bounds__(kStreamThreads) void k_cast(
 // dst[i] = (first ? 0 : dst[i]) + widen(src[i]) over the flat slices of up
 // to kAccumRows gradients: one fp32 rounding per add, as torch's fp32 add_
 // of a widened tensor.  The rows travel by value in the kernel arguments
-// (about 3 KB), so a batch needs no table in device memory.  Block t works
+// (under 4 KB), so a batch needs no table in device memory.  Block t works
 // on tile t of the concatenated rows: row r owns tiles [tile0[r],
 // tile0[r+1]), each of kStreamTile elements in wave order, with the
 // non-temporal hint (the accumulation buffer and the gradient are each
@@ -1405,26 +1405,127 @@ __global__ __launch_bounds__(kStreamThreads) void k_cast(
 // wave sums are added in wave order: bitwise reproducible) and whether any
 // new value is inf/nan.
 constexpr int kAccumRows = MS_ACCUM_ROWS_PER_LAUNCH;
+constexpr int kAccumWideRows = 64;
+constexpr int kAccumBases = 4;
 static_assert(kStreamTile == MS_ACCUM_TILE, "a K5 tile is one statistics slot");
 
-struct AccumLaunch {
-  int64_t tile0[kAccumRows + 1];   // tile0[nrows] = tiles of the launch
-  float* dst[kAccumRows];
-  const void* src[kAccumRows];
-  int64_t numel[kAccumRows];
-  double* ps[kAccumRows];          // per-tile sum of squares, or null
-  uint32_t* pf[kAccumRows];        // per-tile inf/nan flag, or null
-  uint64_t first;                  // bit r: row r overwrites dst
+struct AccumRow {
+  float* dst;
+  const char* src;
+  int64_t n;
+  bool first;                      // overwrite dst
+  double* ps;                      // per-tile sum of squares, or null
+  uint32_t* pf;                    // per-tile inf/nan flag, or null
+};
+
+// The rows of a launch in 24 bytes each: addresses but src's are 32-bit
+// counts of elements (slots) from one of kAccumBases bases, the size is the
+// tiles and the elements of the last one.  A window's gradients go into one
+// buffer per parameter group, so their rows fit, and 148 or 192 gradients take
+// one or two launches, not three (a launch's last blocks leave the chip idle
+// for ~4 us; its arguments take the host 3-4 us): 124M params, two
+// micro-batches of 148 gradients, K5 338 -> 333 us and the window 935 -> 923.
+struct AccumPacked {
+  static constexpr int kRows = kAccumRows;
+  static constexpr uint32_t kTail = 0xfffu, kFirst = 0x1000u, kStats = 0x2000u;
+  static constexpr int kBaseShift = 16;
+  const void* src[kRows];
+  int32_t dst[kRows];              // fp32 elements from dst0[base]
+  int32_t slot[kRows];             // statistics slots from ps0 / pf0[base]
+  uint32_t tile0[kRows + 1];       // tile0[nrows] = tiles of the launch
+  uint32_t bits[kRows];            // elements of the last tile, kFirst, kStats, base
+  float* dst0[kAccumBases];
+  double* ps0[kAccumBases];
+  uint32_t* pf0[kAccumBases];
   int32_t nrows;
   int32_t umode;                   // unscale1 mode of the statistics
   float scale, inv;
+
+  __device__ AccumRow row(int r) const {
+    const uint32_t x = bits[r], b = x >> kBaseShift;
+    AccumRow a;
+    a.dst = dst0[b] + dst[r];
+    a.src = static_cast<const char*>(src[r]);
+    a.n = static_cast<int64_t>(tile0[r + 1] - tile0[r] - 1) * kStreamTile + (x & kTail);
+    a.first = (x & kFirst) != 0;
+    a.ps = (x & kStats) ? ps0[b] + slot[r] : nullptr;
+    a.pf = (x & kStats) ? pf0[b] + slot[r] : nullptr;
+    return a;
+  }
+
+  // Append a row of `tiles` tiles; false when it needs a launch of its own
+  // or one with full addresses.  The bases of a launch are taken as its rows
+  // need them (`nbases` so far).
+  bool add(const ms_accum_row_t& in, int64_t tiles, int& nbases) {
+    if (nrows == kRows || tiles > INT32_MAX - static_cast<int64_t>(tile0[nrows])) return false;
+    const bool stats = in.tile_sumsq != nullptr;
+    for (int b = 0; b <= nbases && b < kAccumBases; ++b) {
+      int64_t d = 0, s = 0, f = 0;
+      if (b == nbases) {
+        dst0[b] = in.dst;
+        ps0[b] = nullptr;
+        ++nbases;
+      } else if (!distance(in.dst, dst0[b], 4, d)) {
+        continue;
+      }
+      if (stats && !ps0[b]) {
+        ps0[b] = in.tile_sumsq;
+        pf0[b] = in.tile_flag;
+      } else if (stats && !(distance(in.tile_sumsq, ps0[b], 8, s) &&
+                            distance(in.tile_flag, pf0[b], 4, f) && s == f)) {
+        continue;
+      }
+      src[nrows] = in.src;
+      dst[nrows] = static_cast<int32_t>(d);
+      slot[nrows] = static_cast<int32_t>(s);
+      bits[nrows] = static_cast<uint32_t>(in.numel - (tiles - 1) * kStreamTile) |
+                    (in.first ? kFirst : 0) | (stats ? kStats : 0) |
+                    static_cast<uint32_t>(b) << kBaseShift;
+      tile0[nrows + 1] = tile0[nrows] + static_cast<uint32_t>(tiles);
+      ++nrows;
+      return true;
+    }
+    return false;
+  }
+
+ private:
+  // (a - b) in units, where it is a whole number of them that fits 32 bits
+  static bool distance(const void* a, const void* b, int64_t unit, int64_t& out) {
+    const int64_t bytes = static_cast<int64_t>(reinterpret_cast<uintptr_t>(a) -
+                                               reinterpret_cast<uintptr_t>(b));
+    out = bytes / unit;
+    return bytes % unit == 0 && out >= INT32_MIN && out <= INT32_MAX;
+  }
 };
-static_assert(kAccumRows <= 64, "one bit of AccumLaunch::first per row");
-static_assert(sizeof(AccumLaunch) <= 4096, "K5 rows must fit in the kernel arguments");
+static_assert(kStreamTile <= AccumPacked::kTail, "a full last tile fits its bits");
+// 256 bytes of the 4 KB kernel argument segment are the implicit arguments
+static_assert(sizeof(AccumPacked) <= 4096 - 256, "K5 rows must fit in the kernel arguments");
+
+// The rows with full addresses, for slices or slots that are far apart.
+struct AccumWide {
+  static constexpr int kRows = kAccumWideRows;
+  int64_t tile0[kRows + 1];        // tile0[nrows] = tiles of the launch
+  float* dst[kRows];
+  const void* src[kRows];
+  int64_t numel[kRows];
+  double* ps[kRows];
+  uint32_t* pf[kRows];
+  uint64_t first;                  // bit r: row r overwrites dst
+  int32_t nrows;
+  int32_t umode;
+  float scale, inv;
+
+  __device__ AccumRow row(int r) const {
+    return {dst[r], static_cast<const char*>(src[r]), numel[r], ((first >> r) & 1u) != 0, ps[r],
+            pf[r]};
+  }
+};
+static_assert(kAccumWideRows <= 64, "one bit of AccumWide::first per row");
+static_assert(sizeof(AccumWide) <= 4096 - 256, "K5 rows must fit in the kernel arguments");
 static_assert(sizeof(ms_accum_row_t) == 48, "ms_accum_row_t layout");
 
-template <class D>
-__global__ __launch_bounds__(kStreamThreads) void k_accumulate(const AccumLaunch L) {
+template <class D, class Launch>
+__global__ __launch_bounds__(kStreamThreads) void k_accumulate(const Launch L) {
   constexpr int kWaves = kStreamThreads / 64;
   __shared__ double wsum[kWaves];
   __shared__ uint32_t wbad[kWaves];
@@ -1441,13 +1542,13 @@ __global__ __launch_bounds__(kStreamThreads) void k_accumulate(const AccumLaunch
       else
         hi = mid - 1;
     }
-    const int r = lo;
-    float* __restrict__ dst = L.dst[r];
-    const char* __restrict__ src = static_cast<const char*>(L.src[r]);
-    const int64_t n = L.numel[r];
-    const bool first = ((L.first >> r) & 1u) != 0;
-    const bool stats = L.ps[r] != nullptr;
-    const int64_t tile = t - L.tile0[r];
+    const AccumRow row = L.row(lo);
+    float* __restrict__ dst = row.dst;
+    const char* __restrict__ src = row.src;
+    const int64_t n = row.n;
+    const bool first = row.first;
+    const bool stats = row.ps != nullptr;
+    const int64_t tile = t - L.tile0[lo];
     const int64_t e0 = tile * kStreamTile;
     const int64_t e1 = (e0 + kStreamTile < n) ? e0 + kStreamTile : n;
     double acc = 0.0;
@@ -1519,8 +1620,8 @@ __global__ __launch_bounds__(kStreamThreads) void k_accumulate(const AccumLaunch
           total += wsum[k];
           flag |= wbad[k];
         }
-        L.ps[r][tile] = total;
-        L.pf[r][tile] = flag;
+        row.ps[tile] = total;
+        row.pf[tile] = flag;
       }
       __syncthreads();   // wsum / wbad are reused by the next tile
     }
@@ -1814,6 +1915,28 @@ int scratch_base(hipStream_t st, unsigned char** out) {
   }
   *out = scratch_ptr[dev];
   return MS_OK;
+}
+
+// One K5 launch over the rows of L
+template <class Launch>
+int launch_accumulate(int32_t src_dtype, Launch& L, int64_t tiles, int umode, float scale,
+                      float inv, hipStream_t st) {
+  L.umode = umode;
+  L.scale = scale;
+  L.inv = inv;
+  const dim3 grid(stream_grid(tiles)), block(kStreamThreads);
+  switch (src_dtype) {
+    case MS_DTYPE_F32:
+      hipLaunchKernelGGL((k_accumulate<DF32, Launch>), grid, block, 0, st, L);
+      break;
+    case MS_DTYPE_F16:
+      hipLaunchKernelGGL((k_accumulate<DF16, Launch>), grid, block, 0, st, L);
+      break;
+    default:
+      hipLaunchKernelGGL((k_accumulate<DBF16, Launch>), grid, block, 0, st, L);
+      break;
+  }
+  return launch_status();
 }
 
 template <class G, class M>
@@ -2151,46 +2274,47 @@ int ms_accumulate_grads(const ms_accum_row_t* rows, int32_t nrows, int32_t src_d
     if ((row.tile_sumsq == nullptr) != (row.tile_flag == nullptr)) return MS_EINVAL;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  AccumLaunch L;
   float inv = 1.0f;
-  L.umode = unscale_mode(unscale, grad_scale, &inv);
-  L.scale = grad_scale;
-  L.inv = inv;
+  const int umode = unscale_mode(unscale, grad_scale, &inv);
+  auto tiles_of = [](const ms_accum_row_t& row) {
+    return row.numel / kStreamTile + (row.numel % kStreamTile != 0);
+  };
   int32_t r = 0;
   while (r < nrows) {
-    // the next launch: up to kAccumRows rows with elements
-    L.nrows = 0;
-    L.first = 0;
+    // the next launch: packed rows, unless full addresses take more
+    AccumPacked P;
+    P.nrows = 0;
+    P.tile0[0] = 0;
+    int nbases = 0;
+    int32_t end = r;
+    for (; end < nrows; ++end)
+      if (rows[end].numel != 0 && !P.add(rows[end], tiles_of(rows[end]), nbases)) break;
+    if (end == nrows || P.nrows >= kAccumWideRows) {
+      r = end;
+      if (P.nrows == 0) break;
+      const int rc = launch_accumulate(src_dtype, P, P.tile0[P.nrows], umode, grad_scale, inv, st);
+      if (rc != MS_OK) return rc;
+      continue;
+    }
+    AccumWide W;
+    W.nrows = 0;
+    W.first = 0;
     int64_t tiles = 0;
-    for (; r < nrows && L.nrows < kAccumRows; ++r) {
+    for (; r < nrows && W.nrows < kAccumWideRows; ++r) {
       const ms_accum_row_t& row = rows[r];
       if (row.numel == 0) continue;
-      const int k = L.nrows++;
-      L.tile0[k] = tiles;
-      L.dst[k] = row.dst;
-      L.src[k] = row.src;
-      L.numel[k] = row.numel;
-      L.ps[k] = row.tile_sumsq;
-      L.pf[k] = row.tile_flag;
-      if (row.first) L.first |= uint64_t(1) << k;
-      tiles += (row.numel + kStreamTile - 1) / kStreamTile;
+      const int k = W.nrows++;
+      W.tile0[k] = tiles;
+      W.dst[k] = row.dst;
+      W.src[k] = row.src;
+      W.numel[k] = row.numel;
+      W.ps[k] = row.tile_sumsq;
+      W.pf[k] = row.tile_flag;
+      if (row.first) W.first |= uint64_t(1) << k;
+      tiles += tiles_of(row);
     }
-    if (L.nrows == 0) break;
-    L.tile0[L.nrows] = tiles;
-    const dim3 grid(stream_grid(tiles));
-    const dim3 block(kStreamThreads);
-    switch (src_dtype) {
-      case MS_DTYPE_F32:
-        hipLaunchKernelGGL(k_accumulate<DF32>, grid, block, 0, st, L);
-        break;
-      case MS_DTYPE_F16:
-        hipLaunchKernelGGL(k_accumulate<DF16>, grid, block, 0, st, L);
-        break;
-      default:
-        hipLaunchKernelGGL(k_accumulate<DBF16>, grid, block, 0, st, L);
-        break;
-    }
-    const int rc = launch_status();
+    W.tile0[W.nrows] = tiles;
+    const int rc = launch_accumulate(src_dtype, W, tiles, umode, grad_scale, inv, st);
     if (rc != MS_OK) return rc;
   }
   return MS_OK;

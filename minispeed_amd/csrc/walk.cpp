@@ -20,6 +20,7 @@
 #include <c10/core/Stream.h>
 #include <c10/core/impl/VirtualGuardImpl.h>
 
+#include <algorithm>
 #include <array>
 #include <cstdint>
 #include <cstring>
@@ -327,7 +328,7 @@ class GradQueue {
   bool empty() const { return entries_.empty(); }
 
   // The queue's content as [(device index, MS_DTYPE_*, rows, gradients)], one
-  // item per device and dtype, in the order of their first entries; rows are
+  // item per device and dtype, group by group in the order they came; rows are
   // ms_accum_row_t records (48 bytes).  The queue is empty afterwards.
   py::list rows() {
     struct Batch {
@@ -337,6 +338,9 @@ class GradQueue {
       py::list grads;
     };
     std::vector<Batch> batches;
+    // a group's rows one after another: K5 takes few buffers in one launch
+    std::stable_sort(entries_.begin(), entries_.end(),
+                     [](const Entry& a, const Entry& b) { return a.group < b.group; });
     for (Entry& e : entries_) {
       const Group& g = groups_[e.group];
       Param& p = groups_[e.group].params[e.index];

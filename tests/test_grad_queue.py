@@ -35,8 +35,9 @@ def test_rows(dtype, code):
         assert q.put(gi, k, grads[gi, k]) == q.AGAIN
     (batch,) = q.rows()
     assert batch[0] == 0 and batch[1] == code and q.empty() and q.rows() == []
-    assert [t.data_ptr() for t in batch[3]] == [t.data_ptr() for t in grads.values()]
-    for row, (gi, k) in zip(_rows(batch), grads):
+    order = sorted(grads, key=lambda x: x[0])       # by group, then as they came
+    assert [t.data_ptr() for t in batch[3]] == [grads[x].data_ptr() for x in order]
+    for row, (gi, k) in zip(_rows(batch), order):
         want = np.array([(ACCUM + (gi << 24) + 4 * OFFSETS[k], grads[gi, k].data_ptr(), SIZES[k], 1, 0,
                           SUMSQ + 8 * TILE0[k], FLAG + 4 * TILE0[k])], dtype=ACCUM_ROW)
         assert row == want[0]
