@@ -32,9 +32,7 @@ class ZeROOptimizer:
         self.rank = comm.get_rank()
         self.adam = FlatAdam(flat_groups, option_groups, zero_stage=zero_stage)
         self.grad_norm: Optional[float] = None
-        self._workspace = Workspace(flat_groups[0].device, len(flat_groups)) if flat_groups else None
-        for g in flat_groups:
-            g.boundary_rows()      # laid out before the first boundary
+        self._workspace: Optional[Workspace] = None
         self.launch_timer: Optional[LaunchTimer] = None  # HIP-event timing hook
         # opt-in fp32 gradient accumulation (contiguous.py); set by the engine
         self.contiguous = None
@@ -105,6 +103,11 @@ class ZeROOptimizer:
         return self.adam.step()
 
     # ------------------------------------------------------ fused boundary
+    def _ws(self) -> Workspace:
+        if self._workspace is None:
+            self._workspace = Workspace(self.flat_groups[0].device, len(self.flat_groups))
+        return self._workspace
+
     def _model_targets(self) -> bool:
         """Ready the parameters for K3's cast into their storage; whether it
         writes them."""
@@ -122,7 +125,7 @@ class ZeROOptimizer:
         Adam step counters advance only for an applied step (the caller
         commits them via :meth:`commit_step`).
         """
-        ws = self._workspace
+        ws = self._ws()
         cur = ws.enter()
         stream = int(cur.device_type), int(cur.device_index), int(cur.stream_id)
         try:
