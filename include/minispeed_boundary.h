@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MS_ABI_VERSION 10
+#define MS_ABI_VERSION 11
 
 /* groups one ms_boundary_scalars_noalloc call can scan, and the tiles
  * (MS_SCAN_TILE flat indices each) of the largest one: its static scratch
@@ -304,7 +304,8 @@ typedef struct ms_boundary_group {
   float *master, *exp_avg, *exp_avg_sq;   /* [dev] fp32, index i at [i - own_begin] */
   ms_adamw_params_t hp;          /* its grad_scale / unscale are K1's as well */
   int32_t scanned;               /* non-zero: the tile slots are filled, no K1 */
-  int32_t reserved;              /* 0 */
+  int32_t update_from_flat;      /* non-zero: K3 reads flat_grad (gradients that share
+                                    its memory, which K1 overwrites) */
 } ms_boundary_group_t;           /* 144 bytes */
 
 /* ms_norm_clip_tiles' arguments after the groups */
@@ -321,8 +322,9 @@ typedef struct ms_norm_args {
 /*
  * The whole boundary in one call: ms_grad_tile_stats of every group that is
  * not scanned, ms_norm_clip_tiles, then ms_fused_adamw (reading the raw
- * gradients) of every group with a non-empty owned range; those functions'
- * checks and results.
+ * gradients, or K1's flat_grad without unscaling it again where
+ * update_from_flat is set) of every group with a non-empty owned range; those
+ * functions' checks and results.
  * groups, stats [host]: ngroups entries; stats[g] are group g's tile slots.
  * events [host, optional]: hipEvent_t pairs recorded around each group's K1
  *   (around nothing where it is scanned), K2 and each K3 that runs.

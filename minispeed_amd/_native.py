@@ -19,7 +19,7 @@ from typing import Optional
 import torch  # noqa: F401  (must precede the dlopen below, see module doc)
 
 LIB_NAME = "libminispeed_boundary.so"
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 DTYPE_F32 = 0
 DTYPE_F16 = 1
@@ -130,7 +130,7 @@ class BoundaryGroup(ctypes.Structure):
         ("exp_avg_sq", ctypes.c_void_p),
         ("hp", AdamWParams),
         ("scanned", ctypes.c_int32),
-        ("reserved", ctypes.c_int32),
+        ("update_from_flat", ctypes.c_int32),
     ]
 
 

@@ -332,6 +332,12 @@ def _tables(gl: GroupLaunch, write_model: bool, gbytes: int, cur: torch.cuda.Str
     return t1, g.table("k3").upload(g.boundary_table(lo, hi, gl.grads, mptrs, gbytes), cur)
 
 
+def _inside(ptrs: np.ndarray, buf: torch.Tensor) -> bool:
+    """Whether any of the addresses lies in ``buf``'s memory."""
+    begin = buf.data_ptr()
+    return bool(((ptrs >= begin) & (ptrs < begin + buf.numel() * buf.element_size())).any())
+
+
 def run_boundary(
     launches: List[GroupLaunch],
     ws: Workspace,
@@ -387,8 +393,14 @@ def run_boundary(
         # K1 writes every element; K3 reads the gradients themselves also
         # then: its unscale rounds exactly as K1's, and 2-byte gradients are
         # 2 B/param less to read than the flat copy (350M fp16 params: K3
-        # 1.77 -> 1.54 ms)
-        b.flat_grad = g.flat_grad_for_overwrite().data_ptr() if materialize_flat_grad else None
+        # 1.77 -> 1.54 ms).  Not where a gradient is a view of the flat
+        # buffer: K1 has unscaled it in place by then
+        b.flat_grad, b.update_from_flat = None, 0
+        if materialize_flat_grad:
+            flat = g.flat_grad_for_overwrite()
+            b.flat_grad = flat.data_ptr()
+            b.update_from_flat = _inside(
+                gl.grads if gl.rows is None else gl.rows.table[:, 2], flat)
         b.master, b.exp_avg, b.exp_avg_sq = (
             master.data_ptr(), gl.exp_avg.data_ptr(), gl.exp_avg_sq.data_ptr())
         b.hp = adamw_params(gl.lr, gl.betas, gl.eps, gl.weight_decay, gl.step,

@@ -2233,6 +2233,8 @@ int ms_boundary_step(const ms_boundary_group_t* groups, const ms_tile_stats_t* s
     return static_cast<int>(hipEventRecord(static_cast<hipEvent_t>(*events++), st));
   };
   int rc = MS_OK;
+  for (int32_t g = 0; g < ngroups; ++g)
+    if (groups[g].update_from_flat && (!groups[g].flat_grad || groups[g].scanned)) return MS_EINVAL;
   for (int32_t g = 0; g < ngroups; ++g) {
     const ms_boundary_group_t& b = groups[g];
     if ((rc = mark()) != MS_OK) return rc;
@@ -2255,8 +2257,14 @@ int ms_boundary_step(const ms_boundary_group_t* groups, const ms_tile_stats_t* s
     const ms_boundary_group_t& b = groups[g];
     if (b.own_end <= b.own_begin) continue;
     if ((rc = mark()) != MS_OK) return rc;
-    rc = ms_fused_adamw(b.master, b.exp_avg, b.exp_avg_sq, nullptr, b.own_segs, b.own_nseg,
-                        b.grad_dtype, b.model_dtype, b.own_begin, b.own_end, &b.hp, norm->out,
+    ms_adamw_params_t hp = b.hp;
+    const float* flat = nullptr;
+    if (b.update_from_flat) {
+      flat = b.flat_grad + b.own_begin;
+      hp.unscale = MS_SCALE_NONE;
+    }
+    rc = ms_fused_adamw(b.master, b.exp_avg, b.exp_avg_sq, flat, b.own_segs, b.own_nseg,
+                        b.grad_dtype, b.model_dtype, b.own_begin, b.own_end, &hp, norm->out,
                         stream);
     if (rc != MS_OK || (rc = mark()) != MS_OK) return rc;
   }

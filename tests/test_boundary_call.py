@@ -11,9 +11,11 @@ import numpy as np
 import pytest
 import torch
 
+import minispeed_amd
 from minispeed_amd import _native
 from minispeed_amd.boundary import LaunchTimer, adamw_params
 from minispeed_amd.flat import FlatParamGroup, _walk
+from minispeed_amd.precision import DynamicLossScaler
 
 INCLUDE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "include")
 STRUCTS = {"ms_boundary_group_t": _native.BoundaryGroup, "ms_norm_args_t": _native.NormArgs,
@@ -221,3 +223,28 @@ def test_recorded_memory_waits_for_the_stream(through_rows, views):
     assert not cur.query()                      # the stream was still busy
     assert not {t.data_ptr() for t in again} & set(held)
     torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lead", [304, 3])
+def test_gradients_that_view_the_flat_gradient(lead):
+    """K1, writing the flat gradient, unscales such gradients in place; K3
+    then takes them from there, once unscaled."""
+    results = []
+    for views in (False, True):
+        gen = torch.Generator(device="cuda").manual_seed(1)
+        params = [torch.nn.Parameter(torch.randn(n, generator=gen, device="cuda"))
+                  for n in (lead, 5000, 77)]
+        engine = minispeed_amd.initialize(model=torch.nn.ParameterList(params), config={
+            "train_micro_batch_size_per_gpu": 1, "dtype": "fp32",
+            "optimizer": {"type": "AdamW", "params": {"lr": 0.1, "eps": 1.0}}})
+        g = engine.flat_groups[0]
+        for p, off, n in zip(g.params, g.layout.offsets, g.layout.numels):
+            grad = torch.randn(n, generator=gen, device="cuda")
+            p.grad = g.grad[off:off + n].copy_(grad) if views else grad
+        scalars = engine.optimizer.boundary_step(DynamicLossScaler(enabled=True, init_scale=8.0), 0.5,
+                                                 materialize_flat_grad=True)
+        results.append([g.data, g.grad, torch.tensor(scalars.norm),
+                        *[engine.optimizer.state[0][k] for k in ("exp_avg", "exp_avg_sq")]])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
