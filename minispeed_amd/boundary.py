@@ -317,10 +317,10 @@ def _tables(gl: GroupLaunch, write_model: bool, gbytes: int, cur: torch.cuda.Str
     if gl.rows is not None:
         # ZeRO-3 placeholders are sized as the parameters unless someone
         # replaced one; the general table looks at what each one covers
-        if gl.rows.models(write_model, g._partitioned) < 0:
+        if gl.rows.models(write_model) < 0:
             t = g.table("k1").upload(gl.rows.table, cur)
             return t, t
-        g.model_pointers()     # raises, unless it is the size
+        g.model_pointers()     # raises, unless it is a placeholder's size
         if gl.grads is None:
             gl.grads = np.zeros(len(g.params) + 1, dtype=np.int64)
             gl.grads[g._whole_rows()[1]] = gl.rows.table[:, 2]

@@ -24,6 +24,7 @@
 #include <array>
 #include <cstdint>
 #include <cstring>
+#include <optional>
 #include <utility>
 #include <vector>
 
@@ -77,21 +78,26 @@ py::tuple grad_pointers(py::list params, py::array_t<int64_t, py::array::c_style
   return py::make_tuple(-1, keep);
 }
 
-// model_pointers(params, device_index, out) -> bad
+// model_pointers(params, device_index, out[, numels]) -> bad
 //   out[k] : data_ptr of params[k] (the cast target), all of the group dtype
-//            (params[0]'s), contiguous and on the device
+//            (params[0]'s), contiguous, on the device and, where numels are
+//            given, of that size
 //   bad    : -1, or the first k that is not
 int64_t model_pointers(py::list params, int64_t device_index,
-                       py::array_t<int64_t, py::array::c_style> out) {
+                       py::array_t<int64_t, py::array::c_style> out,
+                       std::optional<py::array_t<int64_t, py::array::c_style>> numels) {
   const Py_ssize_t n = PyList_GET_SIZE(params.ptr());
-  if (out.size() < n) throw py::value_error("out must have one entry per parameter");
+  if (out.size() < n || (numels && numels->size() != n)) {
+    throw py::value_error("numels / out must have one entry per parameter");
+  }
+  const int64_t* num = numels ? numels->data() : nullptr;
   int64_t* dst = out.mutable_data();
   if (n == 0) return -1;
   const at::ScalarType dtype = unpack(PyList_GET_ITEM(params.ptr(), 0)).scalar_type();
   for (Py_ssize_t k = 0; k < n; ++k) {
     const at::Tensor p = unpack(PyList_GET_ITEM(params.ptr(), k));
     if (!(p.scalar_type() == dtype && p.is_cuda() && p.get_device() == device_index &&
-          p.is_contiguous())) {
+          p.is_contiguous() && (num == nullptr || p.numel() == num[k]))) {
       return static_cast<int64_t>(k);
     }
     dst[k] = reinterpret_cast<int64_t>(p.data_ptr());
@@ -226,8 +232,9 @@ class BoundaryRows {
 
   // Fill the model column with the parameters' storages (write false: with
   // zeros).  -1, or the first parameter that is not contiguous storage of the
-  // group's dtype on its device (sized: or not of its full size).
-  int64_t models(bool write, bool sized) {
+  // group's dtype and of the parameter's full size on its device: K3 writes
+  // whole rows.
+  int64_t models(bool write) {
     std::vector<int64_t> ptrs(numels_.size() + 1, 0);
     check_params();
     if (write && !numels_.empty()) {
@@ -235,7 +242,7 @@ class BoundaryRows {
       for (size_t k = 0; k < numels_.size(); ++k) {
         const at::Tensor p = param(k);
         if (!(p.scalar_type() == dtype && p.is_cuda() && p.get_device() == device_ &&
-              p.is_contiguous() && (!sized || p.numel() == numels_[k]))) {
+              p.is_contiguous() && p.numel() == numels_[k])) {
           return static_cast<int64_t>(k);
         }
         ptrs[k] = reinterpret_cast<int64_t>(p.data_ptr());
@@ -451,7 +458,8 @@ class GradQueue {
 PYBIND11_MODULE(_walk, m) {
   m.doc() = "device addresses of parameter gradients / storages for the boundary tables";
   m.def("grad_pointers", &grad_pointers);
-  m.def("model_pointers", &model_pointers);
+  m.def("model_pointers", &model_pointers, py::arg("params"), py::arg("device_index"),
+        py::arg("out"), py::arg("numels") = py::none());
   m.def("record_streams", &record_streams);
   m.def("release_grads", &release_grads);
   m.def("same_table", &same_table);

@@ -887,12 +887,18 @@ class FlatParamGroup:
     def model_pointers(self) -> np.ndarray:
         """Device address of every parameter's storage (the cast target),
         with a trailing 0 like :meth:`grad_pointers`; every parameter must
-        have the group's dtype, be contiguous and live on its device."""
+        have the group's dtype, be contiguous and live on its device, and be
+        of its full size except as a ZeRO-3 placeholder: the kernels read and
+        write whole parameters through these addresses."""
         ptrs = np.zeros(len(self.params) + 1, dtype=np.int64)
-        bad = _walk().model_pointers(self.params, self._device_index, ptrs)
+        sizes = () if self._partitioned else (self._numels_np,)
+        bad = _walk().model_pointers(self.params, self._device_index, ptrs, *sizes)
         if bad >= 0:
             p = self.params[bad]
             self.model_dtype()   # raises for mixed dtypes
+            if sizes and p.numel() != self._numels[bad]:
+                raise RuntimeError(f"storage of parameter {bad} of its group has {p.numel()} elements, "
+                                   f"expected {self._numels[bad]}")
             raise RuntimeError(
                 f"parameter storage must be contiguous on {self.device}, got {p.device}"
                 + ("" if p.is_contiguous() else " (non-contiguous)"))

@@ -62,8 +62,8 @@ def test_rows_on_the_host():
     rows = _walk().BoundaryRows(params, [3, 0, 5], 0, base, [0, 2, 3])
     rows.set_grads(np.array([11, 12, 13, 0], dtype=np.int64))
     assert rows.table[:, 2].tolist() == [11, 13, 0]
-    assert rows.models(True, False) == 0                 # host storage: the caller's to refuse
-    assert rows.models(False, True) == -1 and rows.table[:, 3].tolist() == [0, 0, 0]
+    assert rows.models(True) == 0                        # host storage: the caller's to refuse
+    assert rows.models(False) == -1 and rows.table[:, 3].tolist() == [0, 0, 0]
     params[2].grad = torch.zeros(5)
     assert rows.grads(1, 0, 0) == 2 and rows.table[:, 2].tolist() == [11, 13, 0]
     with pytest.raises(ValueError):
@@ -76,7 +76,26 @@ def test_rows_on_the_host():
     assert same(base, base.copy()) and not same(base, base[:2])
     params.pop()
     with pytest.raises(ValueError):
-        rows.models(True, False)
+        rows.models(True)
+
+
+def _host_group(sizes):
+    """A group over host tensors, as far as its pointer walk goes."""
+    g = FlatParamGroup.__new__(FlatParamGroup)
+    g.params = [torch.nn.Parameter(torch.zeros(n)) for n in sizes]
+    g.device, g._device_index, g._partitioned = torch.device("cuda:0"), 0, False
+    g._numels, g._numels_np = list(sizes), np.asarray(sizes, dtype=np.int64)
+    return g
+
+
+def test_storage_of_another_size_is_named():
+    g = _host_group((3, 129))
+    for n in (7, 130):
+        g.params[0].data = torch.zeros(n)
+        with pytest.raises(RuntimeError, match=f"parameter 0 of its group has {n} elements, expected 3"):
+            g.model_pointers()
+    with pytest.raises(ValueError):
+        _walk().model_pointers(g.params, 0, np.zeros(3, dtype=np.int64), np.zeros(3, dtype=np.int64))
 
 
 class _Group:
@@ -176,15 +195,15 @@ def test_rows_are_the_pointer_walks():
     both = torch.randn(193, device="cuda").half()     # two gradients of one storage
     params[1].grad, params[2].grad = both[:129], both[129:]
     rows = g.boundary_rows()
-    assert rows.grads(*stream) == -1 and rows.models(True, True) == -1
+    assert rows.grads(*stream) == -1 and rows.models(True) == -1
     want = g.boundary_table(0, g.numel_padded, g.grad_pointers()[0], g.model_pointers())
     assert np.array_equal(rows.table, want)
     params[2].grad = torch.randn(128, device="cuda").half()[::2]
     assert rows.grads(*stream) == 2
     params[1].data = params[1].data[:7].clone()
-    assert rows.models(True, True) == 1 and rows.models(True, False) == -1
+    assert rows.models(True) == 1
     params[1].data = torch.zeros(129, device="cuda")
-    assert rows.models(True, False) == 1
+    assert rows.models(True) == 1
 
 
 @pytest.mark.gpu
@@ -248,3 +267,23 @@ def test_gradients_that_view_the_flat_gradient(lead):
                         *[engine.optimizer.state[0][k] for k in ("exp_avg", "exp_avg_sq")]])
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [7, 130])
+def test_replaced_storage_of_another_size_is_refused(n):
+    """Every kernel that reads or writes whole parameters refuses storage of
+    another size before it is launched."""
+    params = [torch.nn.Parameter(torch.randn(k, device="cuda").half()) for k in (3, 129, 64)]
+    engine = minispeed_amd.initialize(model=torch.nn.ParameterList(params), config={
+        "train_micro_batch_size_per_gpu": 1, "dtype": "fp16",
+        "optimizer": {"type": "AdamW", "params": {"lr": 0.1}}})
+    g = engine.flat_groups[0]
+    before = g.data.clone()
+    params[1].data = torch.zeros(n, dtype=torch.float16, device="cuda")
+    for call in (lambda: engine.optimizer.boundary_step(engine.loss_scaler, None),
+                 g.copy_model_to_flat, g.copy_flat_to_model):
+        with pytest.raises(RuntimeError, match=f"parameter 1 of its group has {n} elements, expected 129"):
+            call()
+    torch.cuda.synchronize()
+    assert torch.equal(g.data, before) and not params[1].any()
