@@ -315,15 +315,15 @@ def _tables(gl: GroupLaunch, write_model: bool, gbytes: int, cur: torch.cuda.Str
     :meth:`FlatParamGroup.boundary_rows`, one each for a shard."""
     g = gl.group
     if gl.rows is not None:
-        # ZeRO-3 placeholders are sized as the parameters unless someone
-        # replaced one; the general table looks at what each one covers
-        if gl.rows.models(write_model) < 0:
-            t = g.table("k1").upload(gl.rows.table, cur)
-            return t, t
-        g.model_pointers()     # raises, unless it is a placeholder's size
-        if gl.grads is None:
-            gl.grads = np.zeros(len(g.params) + 1, dtype=np.int64)
-            gl.grads[g._whole_rows()[1]] = gl.rows.table[:, 2]
+        if write_model and g._partitioned:
+            # K3 writes the shard's buffer, whatever the gathered parameters
+            # view by now; they become its placeholders once K3 is queued
+            gl.rows.set_models(g.shard_pointers())
+        elif gl.rows.models(write_model) >= 0:
+            g.model_pointers()     # says what is wrong with it
+            raise RuntimeError("a parameter changed during the boundary")
+        t = g.table("k1").upload(gl.rows.table, cur)
+        return t, t
     mptrs = g.model_pointers() if write_model else None
     lo, hi = g.own_range
     t1 = g.table("k1").upload(g.boundary_table(0, g.numel_padded, gl.grads, None, gbytes), cur)
@@ -338,7 +338,7 @@ def _inside(ptrs: np.ndarray, buf: torch.Tensor) -> bool:
     return bool(((ptrs >= begin) & (ptrs < begin + buf.numel() * buf.element_size())).any())
 
 
-def run_boundary(
+def launch_boundary(
     launches: List[GroupLaunch],
     ws: Workspace,
     cur: torch.cuda.Stream,
@@ -349,20 +349,20 @@ def run_boundary(
     write_model: bool,
     timer: Optional[LaunchTimer] = None,
     keep: Sequence[Optional[torch.Tensor]] = (),
-) -> _native.StepScalars:
+) -> None:
     """Launch the whole boundary on ``cur`` (the stream ``ws.enter()``
-    returned) and return K2's scalars (one host sync).
+    returned); ``ws.finish_readback()`` then waits for K2's scalars.
 
     One table per group serves K1 and K3 and one call launches every kernel
     (ms_boundary_step): a table and a call per kernel took the host 25 us more
     at every boundary, all of a small model's step.  ``write_model``: K3 casts
-    the updated masters into the parameters' storage.  The function returns
-    once K2's scalars are on the host, which is before K3 has finished: K3
-    runs on ``cur``, so everything queued there afterwards is ordered after
-    it.  ``keep`` holds the tensors behind ``GroupLaunch.grads``; ``cur`` is
-    recorded on each, so the caller may drop them once this returns,
-    whichever stream allocated them (``GroupLaunch.rows`` has recorded it on
-    its own).
+    the updated masters into the parameters' storage.  Whatever can fail (a
+    check, device memory for a table, the tile slots or the flat gradient)
+    does so before the launch, and the gradients and parameters are as they
+    were: the caller releases them after this.  ``keep`` holds the tensors
+    behind ``GroupLaunch.grads``; ``cur`` is recorded on each, so the caller
+    may drop them once this returns, whichever stream allocated them
+    (``GroupLaunch.rows`` has recorded it on its own).
     """
     lib = _native.load()
     scale = float(scaler.loss_scale_factor)
@@ -385,8 +385,9 @@ def run_boundary(
                 f"grad/shard shape mismatch: owned range {hi - lo} vs master {master.numel()}, "
                 f"moments {gl.exp_avg.numel()}/{gl.exp_avg_sq.numel()}"
             )
-        b.model_dtype = _native.ms_dtype(g.params[0].dtype)
-        b.grad_dtype = gdtype = b.model_dtype if gl.grad_dtype is None else gl.grad_dtype
+        dtype = _native.ms_dtype(g.params[0].dtype)
+        b.model_dtype = _native.ms_dtype(g.model_shard.dtype) if g._partitioned else dtype
+        b.grad_dtype = gdtype = dtype if gl.grad_dtype is None else gl.grad_dtype
         (b.segs, b.nseg), (b.own_segs, b.own_nseg) = _tables(
             gl, write_model, 4 if gdtype == _native.DTYPE_F32 else 2, cur)
         b.numel, b.own_begin, b.own_end = g.numel_padded, lo, hi
@@ -433,7 +434,6 @@ def run_boundary(
     rc = lib.ms_boundary_step(ws.groups, ws.tile_stats, len(launches), ctypes.byref(norm), events,
                               cur.cuda_stream)
     _native.check(rc, "ms_boundary_step")
-    return ws.finish_readback()
 
 
 # ------------------------------------------------------------------ utility

@@ -223,9 +223,7 @@ class BoundaryRows {
   // Fill the gradient column with given addresses (one per parameter and a
   // trailing 0 for the padding row).
   void set_grads(py::array_t<int64_t, py::array::c_style> ptrs) {
-    if (ptrs.size() != static_cast<py::ssize_t>(numels_.size()) + 1) {
-      throw py::value_error("one address per parameter and one for the padding");
-    }
+    check_addresses(ptrs);
     held_.clear();
     column(2, ptrs.data());
   }
@@ -252,6 +250,12 @@ class BoundaryRows {
     return -1;
   }
 
+  // Fill the model column with given addresses, as set_grads.
+  void set_models(py::array_t<int64_t, py::array::c_style> ptrs) {
+    check_addresses(ptrs);
+    column(3, ptrs.data());
+  }
+
   // Let go of the gradients (their readers are queued).
   void drop() { held_.clear(); }
 
@@ -261,6 +265,12 @@ class BoundaryRows {
   void check_params() const {
     if (PyList_GET_SIZE(params_.ptr()) != static_cast<Py_ssize_t>(numels_.size())) {
       throw py::value_error("the parameter list changed its length");
+    }
+  }
+
+  void check_addresses(const py::array_t<int64_t, py::array::c_style>& ptrs) const {
+    if (ptrs.size() != static_cast<py::ssize_t>(numels_.size()) + 1) {
+      throw py::value_error("one address per parameter and one for the padding");
     }
   }
 
@@ -470,6 +480,7 @@ PYBIND11_MODULE(_walk, m) {
       .def("grads", &BoundaryRows::grads)
       .def("set_grads", &BoundaryRows::set_grads)
       .def("models", &BoundaryRows::models)
+      .def("set_models", &BoundaryRows::set_models)
       .def("drop", &BoundaryRows::drop);
   py::class_<GradQueue>(m, "GradQueue")
       .def(py::init<>())

@@ -904,6 +904,15 @@ class FlatParamGroup:
                 + ("" if p.is_contiguous() else " (non-contiguous)"))
         return ptrs
 
+    def shard_pointers(self) -> np.ndarray:
+        """The addresses that the parameters have as views of ``model_shard``
+        at world size 1, freed or gathered, with a trailing 0 for the padding
+        row."""
+        size = self.model_shard.element_size()
+        ptrs = np.zeros(len(self.params) + 1, dtype=np.int64)
+        ptrs[:-1] = np.asarray(self.layout.offsets, dtype=np.int64) * size + self.model_shard.data_ptr()
+        return ptrs
+
     def boundary_table(self, lo: int, hi: int, gptrs: Optional[List[int]],
                        mptrs: Optional[List[int]], grad_elem_bytes: Optional[int] = None) -> np.ndarray:
         """Segment table of ``[lo, hi)`` with the given grad / model

@@ -17,7 +17,7 @@ from typing import List, Optional
 import torch
 
 from .. import _native, comm
-from ..boundary import GroupLaunch, LaunchTimer, Workspace, norm_of, run_boundary
+from ..boundary import GroupLaunch, LaunchTimer, Workspace, launch_boundary, norm_of
 from ..flat import FlatParamGroup
 from ..optim.adam import FlatAdam
 
@@ -108,10 +108,15 @@ class ZeROOptimizer:
             self._workspace = Workspace(self.flat_groups[0].device, len(self.flat_groups))
         return self._workspace
 
-    def _model_targets(self) -> bool:
-        """Ready the parameters for K3's cast into their storage; whether it
-        writes them."""
+    def _writes_model(self) -> bool:
+        """Whether K3 casts the updated masters into the parameters' storage."""
         return True
+
+    def _boundary_queued(self) -> None:
+        """Every kernel of the boundary is queued: release ``param.grad``
+        (flat.py:213); what the kernels read is still held."""
+        for g in self.flat_groups:
+            g.release_grads()
 
     def _after_boundary(self, overflow: bool) -> None:
         """Stage-specific follow-up once the scalars are on the host."""
@@ -121,9 +126,11 @@ class ZeROOptimizer:
         """Run flatten/flag/unscale/norm/clip/AdamW/cast for every group as
         K1 -> K2 -> K3 and return the host copy of K2's scalars.
 
-        ``param.grad`` is released for every parameter (flat.py:213).  The
-        Adam step counters advance only for an applied step (the caller
-        commits them via :meth:`commit_step`).
+        ``param.grad`` is released for every parameter (flat.py:213) once the
+        kernels are queued; a boundary that fails before that leaves the
+        gradients and the parameters as they were.  The Adam step counters
+        advance only for an applied step (the caller commits them via
+        :meth:`commit_step`).
         """
         ws = self._ws()
         cur = ws.enter()
@@ -151,15 +158,15 @@ class ZeROOptimizer:
                     step=state["step"] + 1, exp_avg=state["exp_avg"], exp_avg_sq=state["exp_avg_sq"],
                     rows=rows, grads=ptrs, grad_dtype=grad_dtype, tile_stats=tile_stats,
                 ))
-            # release param.grad (flat.py:213); `rows` and `keep` hold what the
-            # kernels read
-            for g in self.flat_groups:
-                g.release_grads()
-            scalars = run_boundary(
+            launch_boundary(
                 launches, ws, cur, scaler=scaler, max_norm=max_norm,
-                materialize_flat_grad=materialize_flat_grad, write_model=self._model_targets(),
+                materialize_flat_grad=materialize_flat_grad, write_model=self._writes_model(),
                 timer=self.launch_timer, keep=keep,
             )
+            self._boundary_queued()
+            # K3 may still run: what is queued on this stream from here on
+            # comes after it
+            scalars = ws.finish_readback()
         finally:
             # (the boundary's stream is recorded on every gradient)
             for g in self.flat_groups:

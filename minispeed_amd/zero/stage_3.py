@@ -89,14 +89,17 @@ class ZeROStage3Optimizer(ZeROOptimizer):
         for g in self.flat_groups:
             g.grad = None
 
-    def _model_targets(self) -> bool:
+    def _writes_model(self) -> bool:
         # not gathered: the reference's free_parameters is a no-op then,
         # nothing is written
+        return self._gathered
+
+    def _boundary_queued(self) -> None:
+        super()._boundary_queued()
         self._boundary_freed = self._gathered
         if self._gathered:
             for g in self.flat_groups:
                 g.dematerialize_params()
-        return self._boundary_freed
 
     def _after_boundary(self, overflow: bool) -> None:
         if self._boundary_freed:
