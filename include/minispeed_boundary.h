@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MS_ABI_VERSION 11
+#define MS_ABI_VERSION 12
 
 /* groups one ms_boundary_scalars_noalloc call can scan, and the tiles
  * (MS_SCAN_TILE flat indices each) of the largest one: its static scratch
@@ -327,11 +327,26 @@ typedef struct ms_norm_args {
  * functions' checks and results.
  * groups, stats [host]: ngroups entries; stats[g] are group g's tile slots.
  * events [host, optional]: hipEvent_t pairs recorded around each group's K1
- *   (around nothing where it is scanned), K2 and each K3 that runs.
+ *   (around nothing where it is scanned), K2 (with the folds of large groups)
+ *   and each K3 that runs.
  */
 int ms_boundary_step(const ms_boundary_group_t* groups, const ms_tile_stats_t* stats,
                      int32_t ngroups, const ms_norm_args_t* norm, void* const* events,
                      void* stream);
+
+/*
+ * Its two halves, for a caller that prepares K3's arguments while K1 runs.
+ * ms_boundary_scan: every K1, then K2.  Of a group it reads segs, nseg,
+ * grad_dtype, numel, own_begin, own_end, flat_grad, scanned and, of hp,
+ * grad_scale and unscale.
+ * ms_boundary_update: every K3, on the stream of the scan; scalars [dev] is
+ * the scan's norm->out.  events: the pairs of its own half.
+ */
+int ms_boundary_scan(const ms_boundary_group_t* groups, const ms_tile_stats_t* stats,
+                     int32_t ngroups, const ms_norm_args_t* norm, void* const* events,
+                     void* stream);
+int ms_boundary_update(const ms_boundary_group_t* groups, int32_t ngroups,
+                       const ms_step_scalars_t* scalars, void* const* events, void* stream);
 
 /*
  * K4 — cast fp32 masters into model-dtype storage: flat [dev] holds index i

@@ -308,28 +308,55 @@ class GroupLaunch:
     # (sum-of-squares slots, flag slots, count) K5 left for the gradients
     # (contiguous mode): folded into the partial sums instead of the K1 scan
     tile_stats: Optional[Tuple[int, int, int]] = None
+    table: Optional[Tuple[int, int]] = None   # _whole_table's
 
 
-def _tables(gl: GroupLaunch, write_model: bool, gbytes: int, cur: torch.cuda.Stream):
-    """K1's and K3's (table address, rows): one table where the group has
-    :meth:`FlatParamGroup.boundary_rows`, one each for a shard."""
+# flat indices that K1 scans for longer than the host takes to upload a table
+# (25 us; 64M fp16 gradients at 5 TB/s)
+_LONG_SCAN = 1 << 26
+
+
+def _whole_table(gl: GroupLaunch, write_model: bool, cur: torch.cuda.Stream) -> Tuple[int, int]:
+    """(address, rows) of the one table of a group with
+    :meth:`FlatParamGroup.boundary_rows`, its model column filled in."""
+    g = gl.group
+    if gl.table is not None:
+        return gl.table
+    if write_model and g._partitioned:
+        # K3 writes the shard's buffer, whatever the gathered parameters view
+        # by now; they become its placeholders once K3 is queued
+        gl.rows.set_models(g.shard_pointers())
+    elif gl.rows.models(write_model) >= 0:
+        g.model_pointers()     # says what is wrong with it
+        raise RuntimeError("a parameter changed during the boundary")
+    gl.table = g.table("k1").upload(gl.rows.table, cur)
+    return gl.table
+
+
+def _scan_table(gl: GroupLaunch, write_model: bool, gbytes: int, cur: torch.cuda.Stream):
+    """K1's (table address, rows).  K1 looks at no model address, so the
+    table with the last boundary's model column serves it before the models
+    are walked: where it is cached, and where K1 runs longer than another
+    upload for K3 takes, should the models have moved (_LONG_SCAN)."""
+    g = gl.group
+    table = g.table("k1")
+    if gl.rows is None:
+        return table.upload(g.boundary_table(0, g.numel_padded, gl.grads, None, gbytes), cur)
+    if g.numel_padded >= _LONG_SCAN:
+        return table.upload(gl.rows.table, cur)
+    return table.find(gl.rows.table, cur) or _whole_table(gl, write_model, cur)
+
+
+def _update_table(gl: GroupLaunch, write_model: bool, gbytes: int, cur: torch.cuda.Stream):
+    """K3's (table address, rows): K1's, or its own for a shard."""
     g = gl.group
     if gl.rows is not None:
-        if write_model and g._partitioned:
-            # K3 writes the shard's buffer, whatever the gathered parameters
-            # view by now; they become its placeholders once K3 is queued
-            gl.rows.set_models(g.shard_pointers())
-        elif gl.rows.models(write_model) >= 0:
-            g.model_pointers()     # says what is wrong with it
-            raise RuntimeError("a parameter changed during the boundary")
-        t = g.table("k1").upload(gl.rows.table, cur)
-        return t, t
-    mptrs = g.model_pointers() if write_model else None
+        return _whole_table(gl, write_model, cur)
     lo, hi = g.own_range
-    t1 = g.table("k1").upload(g.boundary_table(0, g.numel_padded, gl.grads, None, gbytes), cur)
     if hi <= lo:
-        return t1, (None, 0)
-    return t1, g.table("k3").upload(g.boundary_table(lo, hi, gl.grads, mptrs, gbytes), cur)
+        return None, 0
+    mptrs = g.model_pointers() if write_model else None
+    return g.table("k3").upload(g.boundary_table(lo, hi, gl.grads, mptrs, gbytes), cur)
 
 
 def _inside(ptrs: np.ndarray, buf: torch.Tensor) -> bool:
@@ -353,16 +380,18 @@ def launch_boundary(
     """Launch the whole boundary on ``cur`` (the stream ``ws.enter()``
     returned); ``ws.finish_readback()`` then waits for K2's scalars.
 
-    One table per group serves K1 and K3 and one call launches every kernel
-    (ms_boundary_step): a table and a call per kernel took the host 25 us more
-    at every boundary, all of a small model's step.  ``write_model``: K3 casts
-    the updated masters into the parameters' storage.  Whatever can fail (a
-    check, device memory for a table, the tile slots or the flat gradient)
-    does so before the launch, and the gradients and parameters are as they
-    were: the caller releases them after this.  ``keep`` holds the tensors
-    behind ``GroupLaunch.grads``; ``cur`` is recorded on each, so the caller
-    may drop them once this returns, whichever stream allocated them
-    (``GroupLaunch.rows`` has recorded it on its own).
+    K1 and K2 of all groups go out in one call (ms_boundary_scan) as soon as
+    the gradients' addresses are known; K3's table and arguments are made
+    ready behind them, and one call launches every K3 (ms_boundary_update).
+    On an idle GPU the step waits for what comes before K1: with all of it
+    first, K1 of 124M params started 35 us into the step, of 1.3B 50; it
+    starts after 23 and 30 so.  ``write_model``: K3 casts the updated masters
+    into the parameters' storage.  Where this raises (a check, device memory
+    for a table, the tile slots or the flat gradient), the gradients and
+    parameters are as they were: the caller releases them after it.  ``keep``
+    holds the tensors behind ``GroupLaunch.grads``; ``cur`` is recorded on
+    each, so the caller may drop them once this returns, whichever stream
+    allocated them (``GroupLaunch.rows`` records it on its own).
     """
     lib = _native.load()
     scale = float(scaler.loss_scale_factor)
@@ -376,64 +405,71 @@ def launch_boundary(
     ntiles = [0 if done else _native.scan_tiles(gl.group.numel_padded)
               for gl, done in zip(launches, scanned)]
     tsum, tflag = ws.tile_ptrs(sum(ntiles), cur)
+    scale32 = ctypes.c_float(scale).value
+    gbytes = []
     for b, st, gl, done, nt in zip(ws.groups, ws.tile_stats, launches, scanned, ntiles):
         g = gl.group
-        lo, hi = g.own_range
-        master = g.shard
-        if hi > lo and not (master.numel() == gl.exp_avg.numel() == gl.exp_avg_sq.numel() == hi - lo):
-            raise RuntimeError(
-                f"grad/shard shape mismatch: owned range {hi - lo} vs master {master.numel()}, "
-                f"moments {gl.exp_avg.numel()}/{gl.exp_avg_sq.numel()}"
-            )
+        b.numel, (b.own_begin, b.own_end) = g.numel_padded, g.own_range
         dtype = _native.ms_dtype(g.params[0].dtype)
         b.model_dtype = _native.ms_dtype(g.model_shard.dtype) if g._partitioned else dtype
-        b.grad_dtype = gdtype = dtype if gl.grad_dtype is None else gl.grad_dtype
-        (b.segs, b.nseg), (b.own_segs, b.own_nseg) = _tables(
-            gl, write_model, 4 if gdtype == _native.DTYPE_F32 else 2, cur)
-        b.numel, b.own_begin, b.own_end = g.numel_padded, lo, hi
-        # K1 writes every element; K3 reads the gradients themselves also
-        # then: its unscale rounds exactly as K1's, and 2-byte gradients are
-        # 2 B/param less to read than the flat copy (350M fp16 params: K3
-        # 1.77 -> 1.54 ms).  Not where a gradient is a view of the flat
-        # buffer: K1 has unscaled it in place by then
-        b.flat_grad, b.update_from_flat = None, 0
-        if materialize_flat_grad:
-            flat = g.flat_grad_for_overwrite()
-            b.flat_grad = flat.data_ptr()
-            b.update_from_flat = _inside(
-                gl.grads if gl.rows is None else gl.rows.table[:, 2], flat)
-        b.master, b.exp_avg, b.exp_avg_sq = (
-            master.data_ptr(), gl.exp_avg.data_ptr(), gl.exp_avg_sq.data_ptr())
-        b.hp = adamw_params(gl.lr, gl.betas, gl.eps, gl.weight_decay, gl.step,
-                            grad_scale=scale, unscale=unscale)
+        b.grad_dtype = dtype if gl.grad_dtype is None else gl.grad_dtype
+        gbytes.append(4 if b.grad_dtype == _native.DTYPE_F32 else 2)
         b.scanned = done
+        b.flat_grad = g.flat_grad_for_overwrite().data_ptr() if materialize_flat_grad else None
+        b.hp.unscale, b.hp.grad_scale = unscale, scale32
         if done:
             st.sumsq, st.flag, st.ntiles = gl.tile_stats
         else:
+            b.segs, b.nseg = _scan_table(gl, write_model, gbytes[-1], cur)
             st.sumsq, st.flag, st.ntiles = tsum, tflag, nt
             tsum += 8 * nt
             tflag += 4 * nt
-
     norm = ws.norm
     norm.has_clip, norm.max_norm = (0, 0.0) if max_norm is None else (1, float(max_norm))
     norm.scaler_enabled, norm.scale = bool(scaler.enabled), float(scaler.scale)
     norm.good_steps, norm.skipped_steps = int(scaler.good_steps), int(scaler.skipped_steps)
     norm.window = int(scaler.scale_window)
     norm.min_scale, norm.max_scale = float(scaler.min_scale), float(scaler.max_scale)
-    events = None
-    if timer is not None:
-        k3 = sum(gl.group.own_range[1] > gl.group.own_range[0] for gl in launches)
-        events = timer.pairs(["k1"] * len(launches) + ["k2"] + ["k3"] * k3)
+    events = None if timer is None else timer.pairs(["k1"] * len(launches) + ["k2"])
+    ws.readback.arm()
+    rc = lib.ms_boundary_scan(ws.groups, ws.tile_stats, len(launches), ctypes.byref(norm), events,
+                              cur.cuda_stream)
+    _native.check(rc, "ms_boundary_scan")
+    try:
+        for b, gl, size in zip(ws.groups, launches, gbytes):
+            g = gl.group
+            master, n = g.shard, b.own_end - b.own_begin
+            if n > 0 and not (master.numel() == gl.exp_avg.numel() == gl.exp_avg_sq.numel() == n):
+                raise RuntimeError(
+                    f"grad/shard shape mismatch: owned range {n} vs master {master.numel()}, "
+                    f"moments {gl.exp_avg.numel()}/{gl.exp_avg_sq.numel()}"
+                )
+            b.own_segs, b.own_nseg = _update_table(gl, write_model, size, cur)
+            # K3 reads the gradients themselves also when K1 writes the flat
+            # gradient: its unscale rounds exactly as K1's, and 2-byte
+            # gradients are 2 B/param less to read than the flat copy (350M
+            # fp16 params: K3 1.77 -> 1.54 ms).  Not where a gradient is a
+            # view of the flat buffer: K1 unscales it in place
+            b.update_from_flat = materialize_flat_grad and _inside(
+                gl.grads if gl.rows is None else gl.rows.table[:, 2], g.flat_grad_for_overwrite())
+            b.master, b.exp_avg, b.exp_avg_sq = (
+                master.data_ptr(), gl.exp_avg.data_ptr(), gl.exp_avg_sq.data_ptr())
+            b.hp = adamw_params(gl.lr, gl.betas, gl.eps, gl.weight_decay, gl.step,
+                                grad_scale=scale, unscale=unscale)
+        if timer is not None:
+            events = timer.pairs(["k3"] * sum(gl.group.own_range[1] > gl.group.own_range[0]
+                                              for gl in launches))
+        rc = lib.ms_boundary_update(ws.groups, len(launches), norm.out, events, cur.cuda_stream)
+        _native.check(rc, "ms_boundary_update")
+    except BaseException:
+        ws.finish_readback()    # K2's result must not land in the next boundary's
+        raise
     # Gradients may come from another stream (the one backward ran on): once
     # the caller drops them, the caching allocator could hand their memory to
     # that stream while K1 / K3 still read it here.  Recording this stream on
     # them defers the reuse until everything queued here by then has run.
     if keep:
         record_streams(keep, cur)
-    ws.readback.arm()
-    rc = lib.ms_boundary_step(ws.groups, ws.tile_stats, len(launches), ctypes.byref(norm), events,
-                              cur.cuda_stream)
-    _native.check(rc, "ms_boundary_step")
 
 
 # ------------------------------------------------------------------ utility

@@ -1917,6 +1917,15 @@ int scratch_base(hipStream_t st, unsigned char** out) {
   return MS_OK;
 }
 
+// The caller's events, recorded one after another
+struct EventMarks {
+  void* const* next;
+  hipStream_t st;
+  int operator()() {
+    return next ? static_cast<int>(hipEventRecord(static_cast<hipEvent_t>(*next++), st)) : MS_OK;
+  }
+};
+
 // One K5 launch over the rows of L
 template <class Launch>
 int launch_accumulate(int32_t src_dtype, Launch& L, int64_t tiles, int umode, float scale,
@@ -2223,18 +2232,12 @@ int ms_fused_adamw(float* master, float* exp_avg, float* exp_avg_sq,
   return launch_status();
 }
 
-int ms_boundary_step(const ms_boundary_group_t* groups, const ms_tile_stats_t* stats,
+int ms_boundary_scan(const ms_boundary_group_t* groups, const ms_tile_stats_t* stats,
                      int32_t ngroups, const ms_norm_args_t* norm, void* const* events,
                      void* stream) {
   if (ngroups < 0 || (ngroups > 0 && (!groups || !stats)) || !norm) return MS_EINVAL;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  auto mark = [&]() -> int {
-    if (!events) return MS_OK;
-    return static_cast<int>(hipEventRecord(static_cast<hipEvent_t>(*events++), st));
-  };
+  EventMarks mark{events, static_cast<hipStream_t>(stream)};
   int rc = MS_OK;
-  for (int32_t g = 0; g < ngroups; ++g)
-    if (groups[g].update_from_flat && (!groups[g].flat_grad || groups[g].scanned)) return MS_EINVAL;
   for (int32_t g = 0; g < ngroups; ++g) {
     const ms_boundary_group_t& b = groups[g];
     if ((rc = mark()) != MS_OK) return rc;
@@ -2252,7 +2255,16 @@ int ms_boundary_step(const ms_boundary_group_t* groups, const ms_tile_stats_t* s
                           norm->has_clip, norm->max_norm, norm->scaler_enabled, norm->scale,
                           norm->good_steps, norm->skipped_steps, norm->window, norm->min_scale,
                           norm->max_scale, norm->out, norm->out_host, stream);
-  if (rc != MS_OK || (rc = mark()) != MS_OK) return rc;
+  return rc != MS_OK ? rc : mark();
+}
+
+int ms_boundary_update(const ms_boundary_group_t* groups, int32_t ngroups,
+                       const ms_step_scalars_t* scalars, void* const* events, void* stream) {
+  if (ngroups < 0 || (ngroups > 0 && !groups) || !scalars) return MS_EINVAL;
+  EventMarks mark{events, static_cast<hipStream_t>(stream)};
+  int rc = MS_OK;
+  for (int32_t g = 0; g < ngroups; ++g)
+    if (groups[g].update_from_flat && (!groups[g].flat_grad || groups[g].scanned)) return MS_EINVAL;
   for (int32_t g = 0; g < ngroups; ++g) {
     const ms_boundary_group_t& b = groups[g];
     if (b.own_end <= b.own_begin) continue;
@@ -2264,11 +2276,20 @@ int ms_boundary_step(const ms_boundary_group_t* groups, const ms_tile_stats_t* s
       hp.unscale = MS_SCALE_NONE;
     }
     rc = ms_fused_adamw(b.master, b.exp_avg, b.exp_avg_sq, flat, b.own_segs, b.own_nseg,
-                        b.grad_dtype, b.model_dtype, b.own_begin, b.own_end, &hp, norm->out,
-                        stream);
+                        b.grad_dtype, b.model_dtype, b.own_begin, b.own_end, &hp, scalars, stream);
     if (rc != MS_OK || (rc = mark()) != MS_OK) return rc;
   }
   return MS_OK;
+}
+
+int ms_boundary_step(const ms_boundary_group_t* groups, const ms_tile_stats_t* stats,
+                     int32_t ngroups, const ms_norm_args_t* norm, void* const* events,
+                     void* stream) {
+  const int rc = ms_boundary_scan(groups, stats, ngroups, norm, events, stream);
+  if (rc != MS_OK) return rc;
+  return ms_boundary_update(groups, ngroups, norm->out,
+                            events ? events + 2 * (static_cast<int64_t>(ngroups) + 1) : nullptr,
+                            stream);
 }
 
 int ms_accumulate_grads(const ms_accum_row_t* rows, int32_t nrows, int32_t src_dtype,

@@ -175,12 +175,16 @@ bool same_table(py::array_t<int64_t, py::array::c_style> a,
 // place at each boundary.
 class BoundaryRows {
  public:
-  // rows: [n, 4], its first two columns set; index: each row's parameter
-  // (the parameter count: the padding row)
-  BoundaryRows(py::list params, std::vector<int64_t> numels, int64_t device_index,
-               py::array_t<int64_t, py::array::c_style> rows, std::vector<int64_t> index)
-      : params_(std::move(params)), numels_(std::move(numels)), device_(device_index),
-        rows_(std::move(rows)), index_(std::move(index)) {
+  // (taken from an array at once; as std::vector each entry is a Python int)
+  using Ints = py::array_t<int64_t, py::array::c_style | py::array::forcecast>;
+
+  // rows: [n, 4], its first two columns set (copied); index: each row's
+  // parameter (the parameter count: the padding row)
+  BoundaryRows(py::list params, const Ints& numels, int64_t device_index,
+               const py::array_t<int64_t, py::array::c_style>& rows, const Ints& index)
+      : params_(std::move(params)), numels_(numels.data(), numels.data() + numels.size()),
+        device_(device_index), rows_(rows.request()),
+        index_(index.data(), index.data() + index.size()) {
     const int64_t n = static_cast<int64_t>(numels_.size());
     if (rows_.ndim() != 2 || rows_.shape(1) != 4 ||
         rows_.shape(0) != static_cast<py::ssize_t>(index_.size())) {
@@ -193,12 +197,13 @@ class BoundaryRows {
 
   py::array_t<int64_t, py::array::c_style> table() const { return rows_; }
 
-  // Fill the gradient column from param.grad, hold the gradients and record
-  // the stream on them.  -1, or the first parameter whose gradient needs the
-  // slow path; then nothing is held.
+  // Fill the gradient column from param.grad and hold the gradients for
+  // kernels on the given stream.  -1, or the first parameter whose gradient
+  // needs the slow path; then nothing is held.
   int64_t grads(int64_t device_type, int64_t device_index, int64_t stream_id) {
     std::vector<int64_t> ptrs(numels_.size() + 1, 0);
     held_.clear();
+    stream_ = {device_type, device_index, stream_id};
     check_params();
     if (!numels_.empty()) {
       const at::ScalarType dtype = param(0).scalar_type();
@@ -214,8 +219,6 @@ class BoundaryRows {
         held_.push_back(g);
       }
     }
-    StreamRecorder recorder(device_type, device_index, stream_id);
-    for (const at::Tensor& g : held_) recorder.record(g);
     column(2, ptrs.data());
     return -1;
   }
@@ -256,8 +259,14 @@ class BoundaryRows {
     column(3, ptrs.data());
   }
 
-  // Let go of the gradients (their readers are queued).
-  void drop() { held_.clear(); }
+  // Record the stream on the gradients and let go of them (their readers are
+  // queued): nothing before the kernels waits for it.
+  void drop() {
+    if (held_.empty()) return;
+    StreamRecorder recorder(stream_[0], stream_[1], stream_[2]);
+    for (const at::Tensor& g : held_) recorder.record(g);
+    held_.clear();
+  }
 
  private:
   at::Tensor param(size_t k) const { return unpack(PyList_GET_ITEM(params_.ptr(), k)); }
@@ -285,6 +294,7 @@ class BoundaryRows {
   py::array_t<int64_t, py::array::c_style> rows_;
   std::vector<int64_t> index_;
   std::vector<at::Tensor> held_;
+  std::array<int64_t, 3> stream_{};   // device type and index, id
 };
 
 // The gradients queued for K5 (contiguous gradients), one entry per hook call,
@@ -474,8 +484,8 @@ PYBIND11_MODULE(_walk, m) {
   m.def("release_grads", &release_grads);
   m.def("same_table", &same_table);
   py::class_<BoundaryRows>(m, "BoundaryRows")
-      .def(py::init<py::list, std::vector<int64_t>, int64_t,
-                    py::array_t<int64_t, py::array::c_style>, std::vector<int64_t>>())
+      .def(py::init<py::list, const BoundaryRows::Ints&, int64_t,
+                    py::array_t<int64_t, py::array::c_style>, const BoundaryRows::Ints&>())
       .def_property_readonly("table", &BoundaryRows::table)
       .def("grads", &BoundaryRows::grads)
       .def("set_grads", &BoundaryRows::set_grads)

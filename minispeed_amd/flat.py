@@ -221,14 +221,9 @@ class SegmentTable:
         # (host table, device table, streams recorded on it); most recent last
         self._entries: List[Tuple[np.ndarray, torch.Tensor, set]] = []
 
-    def upload(self, table: np.ndarray, stream: Optional[torch.cuda.Stream] = None) -> Tuple[int, int]:
-        """Return (device pointer, row count) of ``table`` for kernels
-        queued on ``stream`` (default: the current stream)."""
-        n = int(table.shape[0])
-        if n == 0:
-            return 0, 0
-        if stream is None:
-            stream = torch.cuda.current_stream(self.device)
+    def find(self, table: np.ndarray, stream: torch.cuda.Stream) -> Optional[Tuple[int, int]]:
+        """(device pointer, row count) of ``table`` where it is cached, for
+        kernels queued on ``stream``."""
         same = _walk().same_table
         for k in range(len(self._entries) - 1, -1, -1):
             host, dev, seen = self._entries[k]
@@ -238,7 +233,20 @@ class SegmentTable:
                 if stream.cuda_stream not in seen:
                     dev.record_stream(stream)
                     seen.add(stream.cuda_stream)
-                return dev.data_ptr(), n
+                return dev.data_ptr(), int(table.shape[0])
+        return None
+
+    def upload(self, table: np.ndarray, stream: Optional[torch.cuda.Stream] = None) -> Tuple[int, int]:
+        """Return (device pointer, row count) of ``table`` for kernels
+        queued on ``stream`` (default: the current stream)."""
+        n = int(table.shape[0])
+        if n == 0:
+            return 0, 0
+        if stream is None:
+            stream = torch.cuda.current_stream(self.device)
+        cached = self.find(table, stream)
+        if cached is not None:
+            return cached
         staging = torch.empty((n, 4), dtype=torch.int64, pin_memory=True)
         staging.numpy()[:] = table
         dev = None
@@ -971,12 +979,13 @@ class FlatParamGroup:
             return None
         if self._native_rows is None:
             base, idx = self._whole_rows()
-            self._native_rows = _walk().BoundaryRows(self.params, self._numels, self._device_index,
-                                                     base.copy(), idx.tolist())
+            self._native_rows = _walk().BoundaryRows(self.params, self._numels_np, self._device_index,
+                                                     base, idx)
         return self._native_rows
 
     def drop_rows(self) -> None:
-        """Let go of the gradients that :meth:`boundary_rows` holds."""
+        """Let go of the gradients that :meth:`boundary_rows` holds (the
+        boundary's stream is recorded on them first)."""
         if self._native_rows is not None:
             self._native_rows.drop()
 

@@ -164,11 +164,12 @@ class ZeROOptimizer:
                 timer=self.launch_timer, keep=keep,
             )
             self._boundary_queued()
+            for g in self.flat_groups:
+                g.drop_rows()
             # K3 may still run: what is queued on this stream from here on
             # comes after it
             scalars = ws.finish_readback()
         finally:
-            # (the boundary's stream is recorded on every gradient)
             for g in self.flat_groups:
                 g.drop_rows()
         overflow = bool(scalars.overflow)

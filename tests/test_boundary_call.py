@@ -12,7 +12,7 @@ import pytest
 import torch
 
 import minispeed_amd
-from minispeed_amd import _native
+from minispeed_amd import _native, boundary
 from minispeed_amd.boundary import LaunchTimer, adamw_params
 from minispeed_amd.flat import FlatParamGroup, _walk
 from minispeed_amd.precision import DynamicLossScaler
@@ -54,6 +54,12 @@ def test_argument_errors_launch_nothing():
     assert call(groups, stats, 1, norm, None, None) == -1          # K1's own checks
     groups.grad_dtype, groups.numel = 1, 5
     assert call(groups, stats, 1, norm, None, None) == -2          # no table
+    update, scalars = lib.ms_boundary_update, ctypes.create_string_buffer(_native.SCALARS_BYTES)
+    assert update(groups, -1, scalars, None, None) == -1
+    assert update(None, 1, scalars, None, None) == -1
+    assert update(groups, 1, None, None, None) == -1
+    groups.update_from_flat = 1                                    # no flat gradient
+    assert update(groups, 1, scalars, None, None) == -1
 
 
 def test_rows_on_the_host():
@@ -287,3 +293,35 @@ def test_replaced_storage_of_another_size_is_refused(n):
             call()
     torch.cuda.synchronize()
     assert torch.equal(g.data, before) and not params[1].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("stage,long_scan,grads_move", [(1, 1 << 26, False), (3, 1 << 26, False),
+                                                        (1, 1, False), (1, 1, True), (1, 1 << 26, True)])
+def test_model_storage_moves(stage, long_scan, grads_move, monkeypatch):
+    """K1 then reads the last boundary's table, or one with its model column;
+    K3 writes the new storage."""
+    monkeypatch.setattr(boundary, "_LONG_SCAN", long_scan)
+    shapes, results = [(3,), (43, 30), (64,)], []
+    for move in (False, True):
+        gen = torch.Generator(device="cuda").manual_seed(2)
+        params = [torch.nn.Parameter(torch.randn(s, generator=gen, device="cuda")) for s in shapes]
+        engine = minispeed_amd.initialize(model=torch.nn.ParameterList(params), config={
+            "train_micro_batch_size_per_gpu": 1, "dtype": "bf16",
+            "optimizer": {"type": "AdamW", "params": {"lr": 0.1}}, "zero_optimization": {"stage": stage}})
+        grads = [torch.randn(s, generator=gen, device="cuda").bfloat16() for s in shapes]
+        for step in range(3):
+            engine.optimizer.gather_parameters()
+            if move and step:
+                for p in params:
+                    p.data = p.data.clone()
+            if grads_move:
+                grads = [t.clone() for t in grads]
+            for p, t in zip(params, grads):
+                p.grad = t
+            engine.micro_steps += 1
+            assert engine.step()
+        engine.optimizer.gather_parameters()
+        results.append([p.detach().clone() for p in params] + [engine.flat_groups[0].shard])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)

@@ -21,8 +21,11 @@ class _Table:
     def __init__(self, fail):
         self.fail = fail
 
+    def find(self, table, stream):
+        return (64, len(table)) if self.fail == "table behind K1" else None
+
     def upload(self, table, stream=None):
-        if self.fail:
+        if self.fail in ("table", "table behind K1"):
             raise torch.OutOfMemoryError("table")
         return 64, len(table)
 
@@ -47,7 +50,7 @@ class _Group(FlatParamGroup):
         self.fail = fail
 
     def table(self, key):
-        return _Table(self.fail == "table")
+        return _Table(self.fail)
 
     def grad_pointers(self):
         grads = [p.grad for p in self.params]
@@ -69,9 +72,13 @@ class _Workspace:
         self.fail, self.norm = fail, _native.NormArgs()
         self.tile_stats, self.groups = (_native.TileStats * 1)(), (_native.BoundaryGroup * 1)()
         self.readback = types.SimpleNamespace(arm=lambda: None)
+        self.waits = 0
 
     def enter(self):
         return _Stream()
+
+    def finish_readback(self):
+        self.waits += 1
 
     def tile_ptrs(self, ntiles, cur):
         if self.fail == "tiles":
@@ -80,8 +87,8 @@ class _Workspace:
 
 
 @pytest.mark.parametrize("stage,fail", [
-    (1, "tiles"), (1, "model"), (1, "moments"), (3, "tiles"), (3, "flat_grad"), (3, "table"),
-    (3, "moments"), (3, "launch")])
+    (1, "tiles"), (1, "model"), (3, "tiles"), (3, "flat_grad"), (3, "table"),
+    (3, "table behind K1"), (3, "moments"), (3, "scan"), (3, "update")])
 def test_nothing_is_released(stage, fail, monkeypatch):
     opt = object.__new__(ZeROStage3Optimizer if stage == 3 else ZeROOptimizer)
     group = _Group(stage, fail)
@@ -93,8 +100,15 @@ def test_nothing_is_released(stage, fail, monkeypatch):
         param_groups=[{"lr": 0.1, "betas": (0.9, 0.99), "eps": 1e-8, "weight_decay": 0.0}],
         state=[{"step": 4, "exp_avg": torch.zeros(n), "exp_avg_sq": torch.zeros(n)}])
     monkeypatch.setattr(boundary, "record_streams", lambda tensors, stream: None)
-    monkeypatch.setattr(boundary._native, "load", lambda: types.SimpleNamespace(
-        ms_boundary_step=lambda *args: -2, ms_error_string=lambda rc: b"no table"))
+    scans = []
+
+    def scan(*args):
+        scans.append(args)
+        return -2 if fail == "scan" else 0
+
+    lib = types.SimpleNamespace(ms_boundary_scan=scan, ms_error_string=lambda rc: b"no table",
+                                ms_boundary_update=lambda *args: -2)
+    monkeypatch.setattr(boundary._native, "load", lambda: lib)
     grads = [torch.randn_like(p) for p in group.params]
     for p, g in zip(group.params, grads):
         p.grad = g
@@ -107,6 +121,9 @@ def test_nothing_is_released(stage, fail, monkeypatch):
     assert [p.data_ptr() for p in group.params] == where
     assert opt._gathered and not opt._boundary_freed
     assert opt.adam.state[0]["step"] == 4
+    # a K2 that was launched is waited for: its result is not the next boundary's
+    behind = fail in ("table behind K1", "moments", "update")
+    assert len(scans) == (behind or fail == "scan") and opt._workspace.waits == behind
 
 
 def test_gathered_parameters_are_written_where_their_placeholders_lie():
