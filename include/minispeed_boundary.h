@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MS_ABI_VERSION 12
+#define MS_ABI_VERSION 13
 
 /* groups one ms_boundary_scalars_noalloc call can scan, and the tiles
  * (MS_SCAN_TILE flat indices each) of the largest one: its static scratch
@@ -394,6 +394,16 @@ typedef struct ms_accum_row {
  * elements one K5 tile (one statistics slot) covers. */
 #define MS_ACCUM_ROWS_PER_LAUNCH 152
 #define MS_ACCUM_TILE 2048
+
+/*
+ * Zero the statistics slots [begin, end) of every range: those that an
+ * earlier window's K5 filled for parameters without a gradient in this one.
+ * ranges [host]: nranges pairs, each inside [0, ntiles) and not empty;
+ * ceil(nranges / MS_CLEAR_RANGES_PER_LAUNCH) launches.
+ */
+#define MS_CLEAR_RANGES_PER_LAUNCH 224
+int ms_clear_tiles(const int64_t* ranges, int32_t nranges, double* tile_sumsq,
+                   uint32_t* tile_flag, int64_t ntiles, void* stream);
 
 /*
  * K5, batched: ms_accumulate_grad for every row of rows[0 .. nrows) [host

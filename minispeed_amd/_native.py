@@ -19,7 +19,7 @@ from typing import Optional
 import torch  # noqa: F401  (must precede the dlopen below, see module doc)
 
 LIB_NAME = "libminispeed_boundary.so"
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 DTYPE_F32 = 0
 DTYPE_F16 = 1
@@ -225,6 +225,7 @@ SIGNATURES = {
     "ms_boundary_update": (ctypes.c_int, [ctypes.POINTER(BoundaryGroup), _I32, _P, _P, _P]),
     "ms_cast_to_model": (ctypes.c_int, [_P, _I64, _I64, _P, _I32, _I32, _P]),
     "ms_accumulate_grad": (ctypes.c_int, [_P, _P, _I32, _I64, _I32, _P]),
+    "ms_clear_tiles": (ctypes.c_int, [_P, _I32, _P, _P, _I64, _P]),
     "ms_accumulate_grads": (ctypes.c_int, [_P, _I32, _I32, _I32, _F, _P]),
     "ms_reduce_tile_stats": (ctypes.c_int, [_P, _P, _I64, _P, _P, _I32, _P]),
     "ms_boundary_scalars_noalloc": (

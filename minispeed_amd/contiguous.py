@@ -223,14 +223,18 @@ class ContiguousGradients:
         w = self._window_unscale
         if w is False or (w is not None and w != unscale_of(float(scale))):
             return None
+        sums, flags = self.tile_sumsq[gi], self.tile_flag[gi]
+        stats = sums.data_ptr(), flags.data_ptr(), int(sums.numel())
         # every K5 of this window wrote all slots of its parameter; what an
-        # earlier window left for the others is cleared here, once (clearing
-        # every slot at every window took two launches a group)
-        for begin, end in self._queue.stale_slots(gi, _native.ACCUM_TILE):
-            self.tile_sumsq[gi][begin:end].zero_()
-            self.tile_flag[gi][begin:end].zero_()
-        return (self.tile_sumsq[gi].data_ptr(), self.tile_flag[gi].data_ptr(),
-                int(self.tile_sumsq[gi].numel()))
+        # earlier window left for the others is cleared here, once, in one
+        # launch (clearing every slot at every window took two a group)
+        stale = self._queue.stale_slots(gi, _native.ACCUM_TILE)
+        if stale:
+            ranges = np.array(stale, dtype=np.int64)
+            _native.check(_native.load().ms_clear_tiles(
+                ranges.ctypes.data, len(ranges), *stats, _native.stream_handle(sums.device)),
+                "ms_clear_tiles")
+        return stats
 
     def next_window(self) -> None:
         """Forget the sums (the boundary consumed them, or zero_grad); queued

@@ -34,6 +34,7 @@
 #include <stdint.h>
 #include <math.h>
 #include <stdlib.h>
+#include <algorithm>
 
 #include <mutex>
 
@@ -1524,6 +1525,27 @@ static_assert(kAccumWideRows <= 64, "one bit of AccumWide::first per row");
 static_assert(sizeof(AccumWide) <= 4096 - 256, "K5 rows must fit in the kernel arguments");
 static_assert(sizeof(ms_accum_row_t) == 48, "ms_accum_row_t layout");
 
+// Clears statistics slots, one range per blockIdx.x.  All latency: a window
+// that leaves out every second of 192 parameters has 96 ranges, which two
+// fills each took 1104 us a window (host), one launch of this 170 (448 with
+// every slot cleared after every window, in Python hooks).
+constexpr int kClearRanges = MS_CLEAR_RANGES_PER_LAUNCH;
+struct ClearLaunch {
+  int64_t begin[kClearRanges], end[kClearRanges];
+  double* sum;
+  uint32_t* flag;
+};
+static_assert(sizeof(ClearLaunch) <= 4096 - 256, "the ranges must fit in the kernel arguments");
+
+__global__ __launch_bounds__(kStreamThreads) void k_clear_tiles(const ClearLaunch L) {
+  const int64_t end = L.end[blockIdx.x];
+  for (int64_t i = L.begin[blockIdx.x] + blockIdx.y * kStreamThreads + threadIdx.x; i < end;
+       i += static_cast<int64_t>(gridDim.y) * kStreamThreads) {
+    L.sum[i] = 0.0;
+    L.flag[i] = 0;
+  }
+}
+
 template <class D, class Launch>
 __global__ __launch_bounds__(kStreamThreads) void k_accumulate(const Launch L) {
   constexpr int kWaves = kStreamThreads / 64;
@@ -2290,6 +2312,32 @@ int ms_boundary_step(const ms_boundary_group_t* groups, const ms_tile_stats_t* s
   return ms_boundary_update(groups, ngroups, norm->out,
                             events ? events + 2 * (static_cast<int64_t>(ngroups) + 1) : nullptr,
                             stream);
+}
+
+int ms_clear_tiles(const int64_t* ranges, int32_t nranges, double* tile_sumsq,
+                   uint32_t* tile_flag, int64_t ntiles, void* stream) {
+  if (nranges < 0 || (nranges > 0 && (!ranges || !tile_sumsq || !tile_flag))) return MS_EINVAL;
+  for (int32_t r = 0; r < nranges; ++r)
+    if (ranges[2 * r] < 0 || ranges[2 * r + 1] <= ranges[2 * r] || ranges[2 * r + 1] > ntiles)
+      return MS_EINVAL;
+  for (int32_t r = 0; r < nranges; r += kClearRanges) {
+    const int n = nranges - r < kClearRanges ? nranges - r : kClearRanges;
+    ClearLaunch L;
+    L.sum = tile_sumsq;
+    L.flag = tile_flag;
+    int64_t longest = 0;
+    for (int k = 0; k < n; ++k) {
+      L.begin[k] = ranges[2 * (r + k)];
+      L.end[k] = ranges[2 * (r + k) + 1];
+      longest = std::max(longest, L.end[k] - L.begin[k]);
+    }
+    const int64_t blocks = (longest + kStreamThreads - 1) / kStreamThreads;
+    hipLaunchKernelGGL(k_clear_tiles, dim3(n, static_cast<uint32_t>(std::min<int64_t>(blocks, 64))),
+                       dim3(kStreamThreads), 0, static_cast<hipStream_t>(stream), L);
+    const int rc = launch_status();
+    if (rc != MS_OK) return rc;
+  }
+  return MS_OK;
 }
 
 int ms_accumulate_grads(const ms_accum_row_t* rows, int32_t nrows, int32_t src_dtype,
