@@ -268,6 +268,28 @@ class BoundaryRows {
     held_.clear();
   }
 
+  // The parameter list is shown to the garbage collector: parameters that
+  // refer to the group (an attribute, a hook over the engine) make a cycle
+  // through this object, and with it unseen the group's buffers stayed.
+  static void collectable(PyHeapTypeObject* heap_type) {
+    PyTypeObject* type = &heap_type->ht_type;
+    type->tp_flags |= Py_TPFLAGS_HAVE_GC;
+    type->tp_traverse = [](PyObject* obj, visitproc visit, void* arg) {
+      Py_VISIT(Py_TYPE(obj));
+      if (py::detail::is_holder_constructed(obj)) {
+        Py_VISIT(py::cast<BoundaryRows&>(py::handle(obj)).params_.ptr());
+      }
+      return 0;
+    };
+    type->tp_clear = [](PyObject* obj) {
+      if (py::detail::is_holder_constructed(obj)) {
+        py::list empty;
+        std::swap(py::cast<BoundaryRows&>(py::handle(obj)).params_, empty);
+      }
+      return 0;
+    };
+  }
+
  private:
   at::Tensor param(size_t k) const { return unpack(PyList_GET_ITEM(params_.ptr(), k)); }
 
@@ -483,7 +505,7 @@ PYBIND11_MODULE(_walk, m) {
   m.def("record_streams", &record_streams);
   m.def("release_grads", &release_grads);
   m.def("same_table", &same_table);
-  py::class_<BoundaryRows>(m, "BoundaryRows")
+  py::class_<BoundaryRows>(m, "BoundaryRows", py::custom_type_setup(&BoundaryRows::collectable))
       .def(py::init<py::list, const BoundaryRows::Ints&, int64_t,
                     py::array_t<int64_t, py::array::c_style>, const BoundaryRows::Ints&>())
       .def_property_readonly("table", &BoundaryRows::table)

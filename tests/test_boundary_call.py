@@ -3,9 +3,11 @@ argument errors and the table's columns on the CPU; on the GPU the one call
 against the entry points it stands for, bit for bit."""
 
 import ctypes
+import gc
 import os
 import shutil
 import subprocess
+import weakref
 
 import numpy as np
 import pytest
@@ -60,6 +62,28 @@ def test_argument_errors_launch_nothing():
     assert update(groups, 1, None, None, None) == -1
     groups.update_from_flat = 1                                    # no flat gradient
     assert update(groups, 1, scalars, None, None) == -1
+
+
+def test_rows_in_a_cycle_are_collected():
+    """Parameters that refer to the engine's objects (an owner attribute, a
+    gradient hook) close a cycle through the rows; it goes when dropped."""
+    class Owner:
+        pass
+
+    for link in ("attribute", "hook"):
+        owner = Owner()
+        owner.params = [torch.nn.Parameter(torch.zeros(3)) for _ in range(2)]
+        for p in owner.params:
+            if link == "attribute":
+                p.owner = owner
+            else:
+                p.register_hook(lambda grad, owner=owner: None)
+        base = np.array([[0, 3, 0, 0], [3, 3, 0, 0]], dtype=np.int64)
+        owner.rows = _walk().BoundaryRows(owner.params, [3, 3], 0, base, [0, 1])
+        gone = weakref.ref(owner)
+        del owner, p
+        gc.collect()
+        assert gone() is None, link
 
 
 def test_rows_on_the_host():
