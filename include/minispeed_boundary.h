@@ -255,9 +255,9 @@ typedef struct ms_tile_stats {
 #define MS_NORM_DIRECT_GROUPS 8
 
 /*
- * ms_reduce_tile_stats of every group, then ms_norm_clip, bit for bit; a
- * group of at most ms_stats_blocks() tiles is read by K2 straight from its
- * tile slots, without the fold's launch.
+ * ms_reduce_tile_stats of every group, then ms_norm_clip, bit for bit; with
+ * nblk == ms_stats_blocks(), a group of at most that many tiles is read by K2
+ * straight from its tile slots, without the fold's launch.
  * groups [host]: ngroups entries.  block_sumsq / block_flag [dev]: workspace
  *   of ngroups x nblk slots (nblk >= ms_stats_blocks()) for the folds.  The
  *   other arguments are ms_norm_clip's.

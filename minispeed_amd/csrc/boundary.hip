@@ -2193,7 +2193,9 @@ int ms_norm_clip_tiles(const ms_tile_stats_t* groups, int32_t ngroups, double* b
   NormTiles direct = {};
   for (int32_t g = 0; g < ngroups; ++g) {
     const ms_tile_stats_t& ts = groups[g];
-    if (g < kNormDirect && ts.ntiles > 0 && ts.ntiles <= kStatsBlocks) {
+    // (the tiles in the slots' places add up as the fold of kStatsBlocks slots
+    // does; more slots a group are added in another order)
+    if (nblk == kStatsBlocks && g < kNormDirect && ts.ntiles > 0 && ts.ntiles <= kStatsBlocks) {
       direct.sum[g] = ts.sumsq;
       direct.flag[g] = ts.flag;
       direct.tiles[g] = static_cast<int32_t>(ts.ntiles);

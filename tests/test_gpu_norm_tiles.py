@@ -91,6 +91,42 @@ def test_norm_from_tiles_equals_fold_and_norm(counts, bad):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("counts", [[1025], [5000, 16384], [40000]])
+@pytest.mark.parametrize("extra", [1024, 16384, 37])
+def test_more_slots_a_group_than_the_fold_needs(counts, extra):
+    """nblk above ms_stats_blocks() spreads the tiles over other slots, so
+    the fold adds them in another order: the result follows it."""
+    lib = _native.load()
+    nb, n = _native.stats_blocks() + extra, len(counts)
+    gen = torch.Generator(device=DEV).manual_seed(extra + sum(counts))
+    # sums of very different sizes: their total depends on the order
+    tiles = [(torch.exp(40 * torch.rand(c, generator=gen, device=DEV, dtype=torch.float64)),
+              torch.zeros(c, dtype=torch.int32, device=DEV)) for c in counts]
+    args = (1, 2.5, 1, 1024.0, 3, 1, 7, 1.0, 2.0 ** 20)
+    ps = torch.empty(n * nb, dtype=torch.float64, device=DEV)
+    pf = torch.empty(n * nb, dtype=torch.int32, device=DEV)
+    want, got = (torch.zeros(_native.SCALARS_BYTES, dtype=torch.uint8, device=DEV) for _ in range(2))
+    for g, (ts, tf) in enumerate(tiles):
+        _native.check(lib.ms_reduce_tile_stats(ts.data_ptr(), tf.data_ptr(), counts[g],
+                                               ps.data_ptr() + 8 * g * nb, pf.data_ptr() + 4 * g * nb,
+                                               nb, None), "fold")
+    _native.check(lib.ms_norm_clip(ps.data_ptr(), pf.data_ptr(), nb, n, *args, want.data_ptr(), None,
+                                   None), "norm")
+    folded = ps.clone(), pf.clone()
+    ps.fill_(7.0)
+    pf.fill_(3)
+    groups = (_native.TileStats * n)(*[_native.TileStats(ts.data_ptr(), tf.data_ptr(), c)
+                                       for c, (ts, tf) in zip(counts, tiles)])
+    _native.check(lib.ms_norm_clip_tiles(groups, n, ps.data_ptr(), pf.data_ptr(), nb, *args,
+                                         got.data_ptr(), None, None), "norm from tiles")
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    # every group was folded into its slots (the fp32 rounding of the sums
+    # hides most changes of order from the scalars)
+    assert torch.equal(ps, folded[0]) and torch.equal(pf, folded[1])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [6144 * 2048 - 5, 6144 * 2048, 6144 * 2048 + 1])
 def test_reading_scan_equals_the_writing_scan_at_the_short_scan_line(n):
     lib = _native.load()
