@@ -89,9 +89,9 @@ class _PinnedSlots:
             free.extend((slab, k) for k in range(self.SLOT, self.SLAB, self.SLOT))
         return dev, slab, off
 
-    def give(self, dev, slab, off, pending) -> None:
+    def give(self, dev, slab, off, ready) -> None:
         # a slot whose kernel may still write is not handed out again
-        if not pending[0] and self._newest.get(dev) is slab:
+        if ready[0] == 1 and self._newest.get(dev) is slab:
             self._free[dev].append((slab, off))
 
 
@@ -112,15 +112,14 @@ class HostReadback:
     device error."""
 
     _READY = _native.StepScalars.ready.offset
-    _pending = [False]   # armed, and K2's result not read yet (each slot has its own)
 
     def __init__(self, patience: float = 5.0):
         dev, slab, off = _SLOTS.take()
-        self._pending = [False]
-        weakref.finalize(self, _SLOTS.give, dev, slab, off, self._pending).atexit = False
         self.host = slab[off:off + _native.SCALARS_BYTES]
         self._bytes = self.host.numpy()
         self._ready = self._bytes[self._READY:self._READY + 4].view(np.uint32)
+        self._ready[0] = 1
+        weakref.finalize(self, _SLOTS.give, dev, slab, off, self._ready).atexit = False
         self.patience = patience
 
     @property
@@ -129,7 +128,11 @@ class HostReadback:
 
     def arm(self) -> None:
         self._ready[0] = 0
-        self._pending[0] = True
+
+    @property
+    def _pending(self) -> np.ndarray:
+        """One truth value: armed, and K2's result not there yet."""
+        return self._ready != 1
 
     def wait(self, stream: int) -> _native.StepScalars:
         ready = self._ready
@@ -144,10 +147,9 @@ class HostReadback:
                 elif now > deadline:
                     _native.hip_check(_native.hip_runtime().hipStreamSynchronize(stream),
                                       "hipStreamSynchronize")
-                    if ready[0] != 1:
+                    if self._pending[0]:
                         raise RuntimeError("the norm/clip kernel's host result did not arrive")
                     break
-        self._pending[0] = False
         return _native.StepScalars.from_buffer_copy(self._bytes.tobytes())
 
 

@@ -334,6 +334,13 @@ def _readback(patience):
     return rb
 
 
+def test_host_readbacks_share_no_state():
+    one, other = _readback(patience=30.0), _readback(patience=30.0)
+    one._ready[0] = other._ready[0] = 1
+    one.arm()
+    assert one._pending[0] and not other._pending[0]
+
+
 def test_host_readback_returns_once_the_ready_word_turns():
     """wait() spins until the kernel's ready word is 1 and then returns the
     struct the kernel wrote before it; arm() clears the word."""
