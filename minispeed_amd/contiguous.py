@@ -49,6 +49,7 @@ minispeed: their segment-table rows carry no gradient address.
 
 from __future__ import annotations
 
+import copy
 import ctypes
 from typing import Callable, List, Optional, Tuple
 
@@ -120,18 +121,38 @@ class ContiguousGradients:
             self._queue.add_group(g._device_index, list(g._numels), list(g.layout.offsets),
                                   tile0.tolist(), accum.data_ptr(),
                                   self.tile_sumsq[-1].data_ptr(), self.tile_flag[-1].data_ptr())
-        self._take, self._slow = self._queue.take, self._queue.SLOW
         # the (unscale, fp32 scale) of this window's flushes; None before the
         # first, False once two differed
         self._window_unscale = None
         # the stream of the last boundary (the sums and slots were read
         # there): a flush on another stream waits for it first
         self._boundary_stream: Optional[torch.cuda.Stream] = None
+        self._register()
+
+    def _register(self) -> None:
+        self._take, self._slow = self._queue.take, self._queue.SLOW
         self._callback_pending = False
         self._handles = []
-        for gi, g in enumerate(groups):
+        for gi, g in enumerate(self.groups):
             for k, p in enumerate(g.params):
                 self._handles.append(p.register_post_accumulate_grad_hook(self._hook(gi, k)))
+
+    def __deepcopy__(self, memo) -> "ContiguousGradients":
+        """The sums so far are copied; a queue and hooks of its own take the
+        gradients of the copied parameters (copies of parameters come without
+        their hooks)."""
+        self.flush()
+        new = memo[id(self)] = object.__new__(type(self))
+        own = {"_queue", "_take", "_slow", "_callback_pending", "_handles", "_boundary_stream"}
+        for name, value in self.__dict__.items():
+            if name not in own:
+                setattr(new, name, copy.deepcopy(value, memo))
+        new._boundary_stream = self._boundary_stream
+        new._queue = self._queue.rebased([
+            (a.data_ptr(), s.data_ptr(), f.data_ptr())
+            for a, s, f in zip(new.accum, new.tile_sumsq, new.tile_flag)])
+        new._register()
+        return new
 
     def _hook(self, gi: int, k: int):
         def hook(param: torch.nn.Parameter) -> None:

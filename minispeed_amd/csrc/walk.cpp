@@ -456,6 +456,21 @@ class GradQueue {
     ++window_;
   }
 
+  // The queue over a copy of the groups' buffers (accum, sumsq, flag of
+  // each): the same windows and slots, nothing queued yet.
+  GradQueue rebased(const std::vector<std::array<int64_t, 3>>& buffers) const {
+    if (buffers.size() != groups_.size() || !entries_.empty()) {
+      throw py::value_error("one (accum, sumsq, flag) per group, and an empty queue");
+    }
+    GradQueue q(*this);
+    for (size_t g = 0; g < buffers.size(); ++g) {
+      q.groups_[g].accum = buffers[g][0];
+      q.groups_[g].sumsq = buffers[g][1];
+      q.groups_[g].flag = buffers[g][2];
+    }
+    return q;
+  }
+
   static constexpr int64_t kNone = -1, kSlow = -2, kAgain = -3;
 
  private:
@@ -526,5 +541,6 @@ PYBIND11_MODULE(_walk, m) {
       .def("rows", &GradQueue::rows)
       .def("pointers", &GradQueue::pointers)
       .def("stale_slots", &GradQueue::stale_slots)
-      .def("next_window", &GradQueue::next_window);
+      .def("next_window", &GradQueue::next_window)
+      .def("rebased", &GradQueue::rebased);
 }

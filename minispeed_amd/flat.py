@@ -624,6 +624,10 @@ class FlatParamGroup:
         self._native_rows = None   # the boundary's table over them
         self._device_index = device.index if device.index is not None else torch.cuda.current_device()
 
+    def __getstate__(self) -> dict:
+        # a copy makes its own boundary table, over its own parameters
+        return {**self.__dict__, "_native_rows": None}
+
     # ------------------------------------------------------------- ranges
     @property
     def master_range(self) -> Range:

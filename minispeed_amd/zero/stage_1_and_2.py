@@ -37,6 +37,10 @@ class ZeROOptimizer:
         # opt-in fp32 gradient accumulation (contiguous.py); set by the engine
         self.contiguous = None
 
+    def __getstate__(self) -> dict:
+        # a copy has scratch (and the word K2 writes on the host) of its own
+        return {**self.__dict__, "_workspace": None}
+
     # ------------------------------------------------------ torch-ish surface
     @property
     def param_groups(self) -> List[dict]:

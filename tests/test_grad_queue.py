@@ -104,3 +104,25 @@ def test_slots_that_an_earlier_window_left():
     q.rows()
     q.next_window()
     assert q.stale_slots(0, 2048) == [(0, 4)]         # neighbours in one range
+
+
+def test_a_copy_of_the_buffers_has_its_own_queue():
+    q = _queue()
+    for k in (0, 2):
+        q.put(0, k, torch.zeros(SIZES[k]))
+    with pytest.raises(ValueError):
+        q.rebased([(8, 16, 24)])                      # something is queued
+    q.rows()
+    with pytest.raises(ValueError):
+        q.rebased([])
+    c, ptrs = q.rebased([(ACCUM + 64, SUMSQ + 64, FLAG + 64)]), np.zeros(3, dtype=np.int64)
+    c.pointers(0, ptrs)
+    assert ptrs.tolist() == [ACCUM + 64, 0, ACCUM + 64 + 4 * OFFSETS[2]]
+    g = torch.zeros(SIZES[2])
+    c.put(0, 2, g)
+    assert q.empty()
+    (batch,) = c.rows()
+    assert _rows(batch).tolist() == [(ACCUM + 64 + 4 * OFFSETS[2], g.data_ptr(), SIZES[2], 0, 0,
+                                      SUMSQ + 64 + 8 * TILE0[2], FLAG + 64 + 4 * TILE0[2])]
+    c.next_window()
+    assert c.stale_slots(0, 2048) == [(0, 4)] and q.stale_slots(0, 2048) == []
