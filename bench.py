@@ -62,13 +62,12 @@ MEASURED_TRAFFIC = {
     "k1/gpt-1.3b/fp16/fused/36.0": 2_639_900_128,
 }
 
-# algorithmic bytes per parameter: (K1, K3) for half / fp32 gradients.  The
-# materialized mode is counted as the unfused data flow, K3 reading the fp32
-# flat gradient; K3 in fact reads the gradients themselves (2 B/param less
-# for half gradients).
+# algorithmic bytes per parameter: (K1, K3) for half / fp32 gradients.  K3
+# reads the gradients themselves in both modes with K1 (the materialized flat
+# gradient is written for the caller).
 BYTES = {
     ("fused", 2): (2, 28),         # K1 read g2 | K3 read g2+p4+m4+v4, write p4+m4+v4+model2
-    ("materialize", 2): (6, 30),   # K1 read g2 write f4 | K3 read f4+12, write 12+2
+    ("materialize", 2): (6, 28),   # K1 read g2 write f4 | K3 as fused
     ("fused", 4): (4, 32),
     ("materialize", 4): (8, 32),
     # contiguous: the accumulation kernel leaves the tile statistics, so the
