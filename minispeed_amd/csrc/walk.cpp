@@ -348,7 +348,7 @@ class GradQueue {
   int64_t take(int64_t gi, int64_t k, py::handle param) {
     Param& p = at(gi, k);
     if (!THPVariable_CheckExact(param.ptr())) return kSlow;
-    const at::Tensor t = THPVariable_Unpack(param.ptr());
+    const at::Tensor& t = THPVariable_Unpack(param.ptr());
     const at::Tensor& g = t.grad();
     if (!g.defined()) return kNone;
     if (g.layout() != at::kStrided || g.numel() != p.numel || !g.is_cuda() ||
@@ -357,8 +357,7 @@ class GradQueue {
       return kSlow;
     }
     if (p.queued) return kAgain;
-    push(gi, k, g);
-    t.mutable_grad().reset();
+    push(gi, k, p, std::move(t.mutable_grad()));
     return queued_;
   }
 
@@ -370,7 +369,7 @@ class GradQueue {
       throw py::value_error("a contiguous f32 / f16 / bf16 gradient of the parameter's size");
     }
     if (p.queued) return kAgain;
-    push(gi, k, g);
+    push(gi, k, p, g);
     return queued_;
   }
 
@@ -497,9 +496,8 @@ class GradQueue {
     return groups_.at(gi).params.at(k);
   }
 
-  void push(int64_t gi, int64_t k, const at::Tensor& g) {
-    Param& p = groups_[gi].params[k];
-    entries_.push_back({gi, k, g, p.seen != window_});
+  void push(int64_t gi, int64_t k, Param& p, at::Tensor g) {
+    entries_.push_back({gi, k, std::move(g), p.seen != window_});
     p.seen = window_;
     p.queued = p.stats = true;
     queued_ += p.numel;
