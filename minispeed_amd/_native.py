@@ -112,7 +112,7 @@ class TileStats(ctypes.Structure):
 
 
 class BoundaryGroup(ctypes.Structure):
-    """``ms_boundary_group_t``: one group of ms_boundary_step."""
+    """``ms_boundary_group_t``: one group of ms_boundary_scan and ms_boundary_update."""
 
     _fields_ = [
         ("segs", ctypes.c_void_p),
@@ -135,7 +135,7 @@ class BoundaryGroup(ctypes.Structure):
 
 
 class NormArgs(ctypes.Structure):
-    """``ms_norm_args_t``: K2's arguments in ms_boundary_step."""
+    """``ms_norm_args_t``: K2's arguments in ms_boundary_scan."""
 
     _fields_ = [
         ("block_sumsq", ctypes.c_void_p),

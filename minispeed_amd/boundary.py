@@ -14,9 +14,9 @@ Replaces the unfused sequence of minispeed's
     (stage 3) free_parameters  stage_3.py:88-110   /
     DynamicLossScaler.update precision.py:50-62        K2 (checked on host)
 
-K3 is gated on the device overflow flag, so one call launches them all and
-does not wait for the host: the only synchronisation is the final copy of the
-``ms_step_scalars_t`` K2 wrote.
+K3 is gated on the device overflow flag, so no launch waits for the host: the
+only synchronisation is the wait for the ``ms_step_scalars_t`` that K2 also
+writes to pinned host memory.
 """
 
 from __future__ import annotations
@@ -262,7 +262,7 @@ class LaunchTimer:
 
     def pairs(self, names: Sequence[str]):
         """An event pair for every name, in order, as the array that
-        ms_boundary_step records."""
+        ms_boundary_scan and ms_boundary_update record."""
         events = (ctypes.c_void_p * (2 * len(names)))()
         for k, name in enumerate(names):
             a, b = (self._pool.pop() if self._pool else self._create() for _ in range(2))
@@ -308,7 +308,7 @@ class GroupLaunch:
     grads: Optional[Sequence[int]]   # (a shard) the address per parameter (0: none)
     grad_dtype: Optional[int] = None   # MS_DTYPE_* of the gradients (default: the params')
     # (sum-of-squares slots, flag slots, count) K5 left for the gradients
-    # (contiguous mode): folded into the partial sums instead of the K1 scan
+    # (contiguous mode): K2's input in the place of what a K1 scan writes
     tile_stats: Optional[Tuple[int, int, int]] = None
     table: Optional[Tuple[int, int]] = None   # _whole_table's
 

@@ -18,8 +18,8 @@ every 2048-element tile of a parameter's slice it writes the fp64 sum of
 squares of the unscaled sums and an inf/nan flag into the tile's slot.
 The last K5 that touched a tile always left the statistics of its current
 sums, and the slots of parameters without a gradient in the window are zeros
-at its boundary, so there the slots are folded into the
-norm's partial sums (``ms_reduce_tile_stats``) and the fp32 sums are not
+at its boundary, so there the norm comes from the slots
+(``ms_norm_clip_tiles``) and the fp32 sums are not
 read a second time: the boundary moves 30 B/param (K3) instead of 34.
 When the loss scale that unscaled the statistics is not the boundary's
 (it changed inside the window), the boundary scans the sums again.
