@@ -1,4 +1,4 @@
-"""ms_boundary_step and the table it is launched with: struct layouts,
+"""ms_boundary_step, its two halves and the table they are launched with: struct layouts,
 argument errors and the table's columns on the CPU; on the GPU the one call
 against the entry points it stands for, bit for bit."""
 

@@ -1,6 +1,6 @@
 """Opt-in contiguous gradients on the GPU.
 
-* K5 (``ms_accumulate_grad``, and batched, ``ms_accumulate_grads``: 150
+* K5 (``ms_accumulate_grad``, and batched, ``ms_accumulate_grads``: 400
   rows, three launches) against the fp32 sum of widened gradients, bit for
   bit, for every dtype, aligned and misaligned slices, ragged sizes,
   inf/nan; the elements between the slices stay untouched;
@@ -13,7 +13,7 @@
   zeros; an overflow skips the step and the next window starts clean;
   ZeRO-3 equals ZeRO-0; flushing the queued gradients inside backward (a
   bucket of one element) equals one flush at the end of backward;
-* the boundary from K5's tile statistics (``ms_reduce_tile_stats``, checked
+* the boundary from K5's tile statistics (the fold, ``ms_reduce_tile_stats``, checked
   on its own against in-order fp64 sums) against the boundary that scans
   the sums again, and the fall-back to that scan when the loss scale
   changed inside a window.
@@ -66,15 +66,16 @@ def test_accumulate_kernel_is_the_fp32_sum(dtype, n, off):
 @pytest.mark.parametrize("dtype,scale_value", [(torch.float16, 1024.0), (torch.bfloat16, 1000.0),
                                                (torch.float32, 3.0)])
 def test_batched_accumulation_is_the_fp32_sum_of_every_row(dtype, scale_value):
-    """150 rows (three launches of 64 / 64 / 22) of ragged sizes, dst slices
+    """400 rows (three launches of up to 152 with elements) of ragged sizes, dst slices
     at every alignment with 3 guard elements between them, some sources one
     element off their alignment, first / add mixed within a launch; the
     tile statistics of the new sums against fp64 on the CPU (power-of-two
     and IEEE-division unscaling), rows without slots leave them alone."""
     from minispeed_amd.contiguous import ACCUM_ROW, accumulate_rows
     rng = np.random.default_rng(7)
-    sizes = rng.choice([0, 1, 3, 4, 2047, 2048, 2049, 4101, 10000], size=150)
-    shifts = rng.integers(0, 4, size=150)          # dst start mod 4
+    sizes = rng.choice([0, 1, 3, 4, 2047, 2048, 2049, 4101, 10000], size=400)
+    assert 2 < np.count_nonzero(sizes) / _native.ACCUM_ROWS_PER_LAUNCH < 3
+    shifts = rng.integers(0, 4, size=400)          # dst start mod 4
     pos, p = [], 8
     for n, sh in zip(sizes, shifts):
         p += (-p + sh) % 4
